@@ -1,0 +1,45 @@
+"""Every engine and control mode on tile sizes at the edges of what a visit
+stages at a time (64-word rows, four rows per slab, the registers that hold a
+tile's internal records), against the oracle bit for bit.  The 9 x 8 grid
+clamps its long edges, so tiles have between 5 and 13 neighbours, and the
+boxes leave some of them out."""
+import numpy as np
+import pytest
+
+import bfnew_amd as bfn
+from helpers import bits, oracle_query
+
+pytestmark = pytest.mark.gpu
+
+CONFIGS = [
+    dict(engine=bfn.JACOBI_PULL, control=bfn.PERSISTENT, sweeps=1, boundary=0),
+    dict(engine=bfn.JACOBI_PULL, control=bfn.CHUNKED, sweeps=0, boundary=0),
+    dict(engine=bfn.DENSE_CHAOTIC_PUSH, control=bfn.PER_ROUND, sweeps=0, boundary=0),
+    dict(engine=bfn.FRONTIER_PUSH, control=bfn.PERSISTENT, sweeps=0, boundary=0),
+    dict(engine=bfn.FRONTIER_PUSH, control=bfn.CHUNKED, sweeps=0, boundary=1, window=4.0),
+]
+
+
+@pytest.mark.parametrize("nodes,block", [(1, 64), (2, 256), (63, 64), (64, 128), (65, 256),
+                                         (129, 64), (257, 256), (301, 512), (513, 256),
+                                         (640, 1024)])
+def test_tile_shapes_bit_exact(device, nodes, block):
+    hg = bfn.HostGraph.synthetic(9, 8, nodes, 7, host_graph=True)
+    view = hg.view()
+    dg = bfn.DeviceGraph(device, hg.layout())
+    qs = hg.synthetic_queries(7, seed=nodes, side_min=2, side_max=8, unbounded_fraction=0.2)
+    tiles = [hg.query_tiles(q) for q in qs]
+    batch = bfn.Batch([[q.source] for q in qs], [[q.target] for q in qs], tiles)
+    want = [oracle_query(view, [q.source], t)[0] for q, t in zip(qs, tiles)]
+    for c in CONFIGS:
+        print("tile shapes", nodes, block, c, flush=True)
+        ws = bfn.Workspace(device)
+        ws.submit(dg, batch, bfn.run_options(engine=c["engine"], control_mode=c["control"],
+                                             rounds_per_chunk=3, block_size=block),
+                  bfn.tuning(tile_sweeps=c["sweeps"], boundary_mode=c["boundary"],
+                             push_window=c.get("window", 0.0)))
+        assert ws.status()[0].converged == 1, c
+        for i in range(len(qs)):
+            assert np.array_equal(bits(ws.distances(i)), bits(want[i])), (c, i)
+        ws.close()
+    dg.close()
