@@ -35,11 +35,16 @@
 //     slot_in[]/slot_out[]  slot of each in/out-neighbour tile for q, or NONE
 //     stamp[s]       1 + last round s was queued for (dedups the work lists)
 //     lists[3][S]    round-robin work lists; list r%3 is consumed in round r,
-//                    list (r+1)%3 is filled, list (r+2)%3 is reset.
+//                    list (r+1)%3 is filled, list (r+2)%3 is reset.  A list
+//                    is cut into kQueueClasses parts, part x for the slots
+//                    with s % kQueueClasses == x (each at most once per
+//                    round, so the parts together hold exactly S entries)
+//     queue[]        per list, the count of each part and the claim counters
 #pragma once
 
 #include <hip/hip_runtime.h>
 
+#include <cstddef>
 #include <cstdint>
 
 namespace bfn {
@@ -70,6 +75,17 @@ constexpr std::uint32_t kBarrierGroups = 8;
 constexpr std::uint32_t kMaxArrivalGroups = 64;  // arrival counters in DevControl
 constexpr std::uint32_t kArrivalGroups = 32;     // used by the relaxation kernels
 constexpr std::uint32_t kBarrierStride = 32;  // words: one 128-byte line per group
+
+// Work-list counters.  Atomics on one address are served one after another
+// at the memory side, 11.4 ns each on MI355X however many workgroups issue
+// them (5.7 ns over 2 addresses, 1.8 over 8, 0.26 over 64): with one append
+// counter and one claim counter per round, 128x128x512 tiles and 256 queries
+// spent ~5 of 15 ms, and 32 point-Jacobi lanes nearly all of a round, queuing
+// on them.  So a list has one append counter per class of slots and one claim
+// counter per group of workgroups, each on a line of its own; 64 of each, so
+// that one wave reads a round's counts at once.
+constexpr std::uint32_t kQueueClasses = 64;
+constexpr std::uint32_t kQueueWords = 2u * 3u * kQueueClasses * kBarrierStride;
 
 enum Engine : std::uint32_t { kJacobiPull = 0, kDensePush = 1, kFrontierPush = 2 };
 
@@ -125,19 +141,15 @@ struct DevGraph {
 // Control block; lives in device memory, one per workspace.
 // Words that workgroups hit with atomics or polls during a round sit on
 // 128-byte lines of their own: agent-scope atomics and coherent loads of one
-// line are served one after another at the memory side, so enqueues
-// (list_count), claims (claim) and the barrier polls of finished workgroups
-// (barrier_generation) would otherwise queue behind each other.
+// line are served one after another at the memory side.  The work-list
+// counters are a buffer of their own (DevBatch::queue).  What the host reads
+// back comes first; a control copy ends at kControlHead.
 struct DevControl {
   std::uint32_t round;            // next round to execute
   std::uint32_t done;
   std::uint32_t stop_reason;
   std::uint32_t error_bits;
   std::uint32_t rounds_executed;
-  alignas(128) std::uint32_t list_count[3];
-  alignas(128) std::uint32_t claim[3];
-  alignas(128) std::uint32_t barrier_count;
-  alignas(128) std::uint32_t barrier_generation;
   alignas(128) unsigned long long items_processed;
   unsigned long long edges_examined;
   unsigned long long atomic_attempts;
@@ -148,11 +160,13 @@ struct DevControl {
   unsigned long long closure_sweeps;     // tile-closure sweeps (one per block pass)
   unsigned long long candidates;         // candidate labels computed by the visits
   unsigned long long phase_cycles[kPhaseCount];  // summed over workgroups
+  alignas(128) std::uint32_t barrier_count;
+  alignas(128) std::uint32_t barrier_generation;
   // Slot-order claims: the compacted list of the round is cut into one
   // segment per XCD group, [seg_begin[x], seg_begin[x+1]) (read once per
   // round launch); seg_claim[x * kBarrierStride] is the next unclaimed
   // position of segment x, each counter on its own 128-byte line.
-  std::uint32_t seg_begin[kBarrierGroups + 1];
+  alignas(128) std::uint32_t seg_begin[kBarrierGroups + 1];
   alignas(128) std::uint32_t seg_claim[kBarrierGroups * kBarrierStride];
   // Push window: rounds visit the queued slots whose priority (smallest
   // label pushed in since their last visit) is at most `window_limit`.
@@ -165,6 +179,11 @@ struct DevControl {
   // workgroups (blockIdx % G), each on its own 128-byte line.
   alignas(128) std::uint32_t group_arrivals[kMaxArrivalGroups * kBarrierStride];
 };
+constexpr std::size_t kControlHead = offsetof(DevControl, barrier_count);
+// What workspace estimates and the static scratch count for a batch's control
+// block.
+constexpr std::size_t kControlBytes = 13312;
+static_assert(sizeof(DevControl) <= kControlBytes, "control block within its estimate");
 
 // What a visit of slot s needs before it can load any label: written once
 // per batch by the preparation kernel, so a visit starts with one 64-byte
@@ -224,7 +243,8 @@ struct DevBatch {
   std::uint32_t* lists;                 // [3*S]
   std::uint32_t* dist;                  // float bits pool
   std::uint32_t* last_change;           // [Q] 1 + last round with a decrease
-  std::uint32_t* pending;               // [Q] queued work items of q, or null
+  std::uint32_t* pending;               // [Q] 1 + last round q has work queued for, or null
+  std::uint32_t* queue;                 // kQueueWords: append and claim counters of the lists
   DevControl* control;
 };
 
@@ -294,50 +314,35 @@ __device__ __forceinline__ void atomic_or_agent(std::uint32_t* p, std::uint32_t 
 __device__ __forceinline__ float as_float(std::uint32_t b) { return __uint_as_float(b); }
 __device__ __forceinline__ std::uint32_t as_bits(float f) { return __float_as_uint(f); }
 
-// Queues slot for `round` once: the stamp dedups, the list append claims a
-// position, and the query's pending work (when tracked) counts the item.
-__device__ __forceinline__ void enqueue(const DevBatch& b, std::uint32_t slot,
-                                        std::uint32_t round) {
-  if (b.ordered) {
-    atomic_or_agent(&b.active[slot >> 5], 1u << (slot & 31u));
-    return;
-  }
-  const std::uint32_t tag = round + 1;
-  if (atomic_max_agent(&b.stamp[slot], tag) < tag) {
-    const std::uint32_t li = round % 3;
-    const std::uint32_t pos = atomic_add_agent(&b.control->list_count[li], 1u);
-    b.lists[static_cast<std::size_t>(li) * b.slot_count + pos] = slot;
-    if (b.pending) atomic_add_agent(&b.pending[b.slot_query[slot]], 1u);
-  }
+// Append counter of class x and claim counter of group x of list li.
+__device__ __forceinline__ std::uint32_t* list_count(const DevBatch& b, std::uint32_t li, std::uint32_t x) {
+  return b.queue + (li * kQueueClasses + x) * kBarrierStride;
+}
+__device__ __forceinline__ std::uint32_t* list_claim(const DevBatch& b, std::uint32_t li, std::uint32_t x) {
+  return b.queue + ((3u + li) * kQueueClasses + x) * kBarrierStride;
+}
+// First entry of class x within a list.
+__device__ __forceinline__ std::uint32_t class_begin(std::uint32_t slots, std::uint32_t x) {
+  return x * (slots / kQueueClasses) + min(x, slots % kQueueClasses);
 }
 
-// Wave-wide enqueue: every lane of the wave calls it in uniform control
-// flow; lanes with `want` queue `slot` for `round`.  The stamps dedup per
-// slot as in enqueue(), and the lanes that queue a slot first share one
-// list-position claim per wave (one atomic on the list counter instead of
-// one per slot).
-__device__ __forceinline__ void enqueue_wave(const DevBatch& b, std::uint32_t slot, bool want,
-                                             std::uint32_t round) {
+// Queues slot for `round` once: the stamp dedups and the append claims a
+// position in the slot's class of the list.  Returns whether this call queued
+// it.  A query's pending mark (when tracked) is stored by the caller: every
+// writer of a round stores the same value.
+__device__ __forceinline__ bool enqueue(const DevBatch& b, std::uint32_t slot, std::uint32_t round) {
   if (b.ordered) {
     // A bit per slot: setting it twice queues the slot once, and no lane
     // waits for a returned value.
-    if (want) atomic_or_agent(&b.active[slot >> 5], 1u << (slot & 31u));
-    return;
+    atomic_or_agent(&b.active[slot >> 5], 1u << (slot & 31u));
+    return true;
   }
   const std::uint32_t tag = round + 1;
-  const std::uint32_t lane = threadIdx.x & 63u;
-  const bool first = want && atomic_max_agent(&b.stamp[slot], tag) < tag;
-  const unsigned long long m = __ballot(first);
-  if (m == 0) return;
-  const std::uint32_t li = round % 3;
-  std::uint32_t base = 0;
-  if (lane == 0) base = atomic_add_agent(&b.control->list_count[li], static_cast<std::uint32_t>(__popcll(m)));
-  base = __shfl(base, 0);
-  if (first) {
-    const std::uint32_t rank = static_cast<std::uint32_t>(__popcll(m & ((1ull << lane) - 1ull)));
-    b.lists[static_cast<std::size_t>(li) * b.slot_count + base + rank] = slot;
-    if (b.pending) atomic_add_agent(&b.pending[b.slot_query[slot]], 1u);
-  }
+  if (atomic_max_agent(&b.stamp[slot], tag) >= tag) return false;
+  const std::uint32_t li = round % 3, x = slot % kQueueClasses;
+  const std::uint32_t pos = class_begin(b.slot_count, x) + atomic_add_agent(list_count(b, li, x), 1u);
+  b.lists[static_cast<std::size_t>(li) * b.slot_count + pos] = slot;
+  return true;
 }
 
 // Neighbour entries of a visit's LDS table, and the words of LDS one
@@ -360,6 +365,9 @@ __host__ __device__ constexpr std::size_t relax_lds_words(std::uint32_t max_v, s
 constexpr std::uint32_t kBarrierSpinLimit = 1u << 23;
 constexpr std::uint32_t kProbeSpinLimit = 1u << 16;  // co-residency probe launches
 constexpr std::uint32_t kErrorBarrierTimeout = 8u;
+// Before its workgroup barrier every wave waits for its own stores: thread 0
+// writes the L2 back for the whole workgroup, and a workgroup barrier alone
+// does not wait for the other waves' stores to get there.
 
 __device__ __forceinline__ bool barrier_wait(DevControl* c, std::uint32_t gen, std::uint32_t limit) {
   for (std::uint32_t spins = 0; load_agent(&c->barrier_generation) == gen; ++spins) {
@@ -377,6 +385,7 @@ __device__ __forceinline__ bool barrier_wait(DevControl* c, std::uint32_t gen, s
 // and advances the generation that the others wait on.
 __device__ __forceinline__ bool grid_barrier_flat(DevControl* c, std::uint32_t blocks,
                                                   std::uint32_t limit = kBarrierSpinLimit) {
+  __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   bool ok = true;
   if (threadIdx.x == 0) {
@@ -409,6 +418,7 @@ template <std::uint32_t G = kArrivalGroups>
 __device__ __forceinline__ bool grid_barrier_grouped(DevControl* c, std::uint32_t blocks,
                                                      std::uint32_t limit = kBarrierSpinLimit) {
   static_assert(G % kBarrierGroups == 0 && G <= kMaxArrivalGroups, "arrival groups");
+  __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   bool ok = true;
   if (threadIdx.x == 0) {

@@ -160,7 +160,7 @@ struct bfn_workspace_s {
   hipStream_t stream = nullptr;
   std::uint64_t budget = 0;
   // batch metadata in one device buffer + separately grown state
-  DeviceBuffer meta, slot_in, slot_out, slot_out_off, slot_desc, stamp, prio, lists, pool, last_change, control,
+  DeviceBuffer meta, slot_in, slot_out, slot_out_off, slot_desc, stamp, prio, lists, pool, last_change, control, queue,
       status, relax,
       scratch_v, paths_summary, paths_len, paths_off, frames, onpath, clean, arena_v, arena_l,
       arena_e, occupancy, region_off;
@@ -823,7 +823,7 @@ std::uint64_t batch_bytes(const BatchPlanHost& p, std::uint64_t meta_bytes) {
   return meta_bytes + 4ull * (p.in_total + p.out_total) + 8ull * p.out_total +
          (20ull + sizeof(SlotDesc)) * p.S +
          4ull * p.pool_words + 4ull * p.Q * 2 + sizeof(QueryStatusDev) * p.Q + 8ull * p.Q +
-         sizeof(DevControl);
+         kControlBytes;
 }
 
 // Sets up the DevBatch view over the workspace buffers.
@@ -866,6 +866,7 @@ void bind_view(bfn_workspace ws, const BatchPlanHost& p, const std::size_t* seg,
   b.dist = ws->pool.as<std::uint32_t>();
   b.last_change = ws->last_change.as<std::uint32_t>();
   b.pending = nullptr;
+  b.queue = ws->queue.as<std::uint32_t>();
   b.control = ws->control.as<DevControl>();
 }
 
@@ -893,7 +894,7 @@ int32_t run_resident_batch(bfn_workspace ws) {
       e = hipMemcpyAsync(ws->h_status.ptr, ws->status.ptr, sizeof(QueryStatusDev) * b.query_count,
                          hipMemcpyDeviceToHost, s);
     if (e == hipSuccess)
-      e = hipMemcpyAsync(ws->h_control.ptr, ws->control.ptr, sizeof(DevControl),
+      e = hipMemcpyAsync(ws->h_control.ptr, ws->control.ptr, kControlHead,
                          hipMemcpyDeviceToHost, s);
     return e;
   };
@@ -923,7 +924,7 @@ int32_t run_resident_batch(bfn_workspace ws) {
         e = relax_launch(ws->block, false, false, ws->grid, ws->lds_bytes, ws->max_v,
                          ws->work_words, g->view, b, s);
       if (e == hipSuccess)
-        e = hipMemcpyAsync(ws->h_control.ptr, ws->control.ptr, sizeof(DevControl),
+        e = hipMemcpyAsync(ws->h_control.ptr, ws->control.ptr, kControlHead,
                            hipMemcpyDeviceToHost, s);
       hipGraph_t captured = nullptr;
       const hipError_t end = hipStreamEndCapture(s, &captured);
@@ -951,7 +952,7 @@ int32_t run_resident_batch(bfn_workspace ws) {
         BFN_HIP(relax_launch(ws->block, false, false, ws->grid, ws->lds_bytes, ws->max_v,
                              ws->work_words, g->view, b, s));
       ws->launches += 2ull * chunk;
-      BFN_HIP(hipMemcpyAsync(ws->h_control.ptr, ws->control.ptr, sizeof(DevControl),
+      BFN_HIP(hipMemcpyAsync(ws->h_control.ptr, ws->control.ptr, kControlHead,
                              hipMemcpyDeviceToHost, s));
       BFN_HIP(hipStreamSynchronize(s));
       ++ws->host_checks;
@@ -978,7 +979,7 @@ int32_t run_resident_batch(bfn_workspace ws) {
         BFN_HIP(relax_launch(ws->block, false, false, ws->grid, ws->lds_bytes, ws->max_v,
                              ws->work_words, g->view, b, s));
       ws->launches += 2ull * chunk;
-      BFN_HIP(hipMemcpyAsync(ws->h_control.ptr, ws->control.ptr, sizeof(DevControl),
+      BFN_HIP(hipMemcpyAsync(ws->h_control.ptr, ws->control.ptr, kControlHead,
                              hipMemcpyDeviceToHost, s));
       BFN_HIP(hipStreamSynchronize(s));
       ++ws->host_checks;
@@ -1100,6 +1101,7 @@ int32_t bfn_batch_submit(bfn_workspace ws, bfn_graph graph, const bfn_batch_desc
   BFN_HIP(ws->pool.reserve(4ull * std::max<std::uint64_t>(p.pool_words, 1)));
   BFN_HIP(ws->last_change.reserve(4ull * Q));
   BFN_HIP(ws->control.reserve(sizeof(DevControl)));
+  BFN_HIP(ws->queue.reserve(4ull * kQueueWords));
   BFN_HIP(ws->status.reserve(sizeof(QueryStatusDev) * Q));
   BFN_HIP(ws->relax.reserve(8ull * Q));
   BFN_HIP(ws->h_status.reserve(sizeof(QueryStatusDev) * Q));

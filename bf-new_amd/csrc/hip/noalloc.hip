@@ -34,20 +34,28 @@ constexpr int kMaxDevices = 64;
 
 __device__ __align__(256) std::uint32_t scratch[kStaticScratchBytes / 4];
 
-// Device address of each GPU's `scratch`, looked up once per device with
-// that device current (host code never uses the array's name as an address).
+// The work-list counters, 48 KiB beside the scratch: a batch that fills the
+// scratch to its last segment still has them.
+__device__ __align__(256) std::uint32_t queue_counters[kQueueWords];
+
+// Device addresses of each GPU's arrays, looked up once per device with
+// that device current (host code never uses an array's name as an address).
 std::mutex g_scratch_mutex;
 void* g_scratch_ptr[kMaxDevices] = {};
+void* g_queue_ptr[kMaxDevices] = {};
 
-hipError_t scratch_address(int ordinal, void** out) {
+hipError_t scratch_address(int ordinal, void** out, void** queue) {
   std::lock_guard<std::mutex> lock(g_scratch_mutex);
   if (!g_scratch_ptr[ordinal]) {
-    void* p = nullptr;
-    const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+    void *p = nullptr, *q = nullptr;
+    hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+    if (e == hipSuccess) e = hipGetSymbolAddress(&q, HIP_SYMBOL(queue_counters));
     if (e != hipSuccess) return e;
+    g_queue_ptr[ordinal] = q;
     g_scratch_ptr[ordinal] = p;
   }
   *out = g_scratch_ptr[ordinal];
+  *queue = g_queue_ptr[ordinal];
   return hipSuccess;
 }
 
@@ -194,7 +202,7 @@ int32_t bfn_batch_run_static(bfn_graph graph, const bfn_batch_desc* d, const bfn
     at = align256(at + std::max<std::size_t>(bytes, 4));
     return here;
   };
-  const std::size_t o_control = take(sizeof(DevControl));
+  const std::size_t o_control = take(kControlBytes);
   const std::size_t o_status = take(sizeof(QueryStatusDev) * Q);
   const std::size_t o_targets = take(4ull * nt);
   const std::size_t o_tile_off = take(4ull * (Q + 1));
@@ -240,8 +248,8 @@ int32_t bfn_batch_run_static(bfn_graph graph, const bfn_batch_desc* d, const bfn
   if (o->grid_policy == 1) grid = std::min(grid, o->blocks_per_wgp * gh.cu_count);
   grid = std::max(grid, 1u);
 
-  void* base_ptr = nullptr;
-  BFN_HIP_STATIC(scratch_address(gh.ordinal, &base_ptr));
+  void *base_ptr = nullptr, *queue_ptr = nullptr;
+  BFN_HIP_STATIC(scratch_address(gh.ordinal, &base_ptr, &queue_ptr));
   char* m = static_cast<char*>(base_ptr);
   auto u32 = [&](std::size_t off) { return reinterpret_cast<std::uint32_t*>(m + off); };
   DevBatch b{};
@@ -281,6 +289,7 @@ int32_t bfn_batch_run_static(bfn_graph graph, const bfn_batch_desc* d, const bfn
   b.dist = u32(o_pool);
   b.last_change = u32(o_last);
   b.pending = nullptr;
+  b.queue = static_cast<std::uint32_t*>(queue_ptr);
   b.control = reinterpret_cast<DevControl*>(m + o_control);
 
   const hipStream_t s = gh.stream;

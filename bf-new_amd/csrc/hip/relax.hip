@@ -9,21 +9,30 @@
 
 namespace bfn {
 
-__global__ void relax_advance_kernel(DevBatch b) {
+// One wave: lane x looks after class x of the lists.
+__global__ __launch_bounds__(64) void relax_advance_kernel(DevBatch b) {
+  static_assert(kQueueClasses == 64, "one lane per class");
   DevControl* c = b.control;
   if (c->done) return;
+  const std::uint32_t lane = threadIdx.x;
   const std::uint32_t r = c->round;
-  const std::uint32_t n = c->list_count[r % 3];
-  if (b.instrumentation && n > c->max_list) c->max_list = n;
-  c->list_count[(r + 2) % 3] = 0;
-  c->claim[(r + 2) % 3] = 0;
+  const bool queued = *list_count(b, (r + 1) % 3, lane) != 0;
+  const bool any = __ballot(queued) != 0;
+  if (b.instrumentation) {
+    std::uint32_t n = *list_count(b, r % 3, lane);
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off);
+    if (lane == 0 && n > c->max_list) c->max_list = n;
+  }
+  *list_count(b, (r + 2) % 3, lane) = 0;
+  *list_claim(b, (r + 2) % 3, lane) = 0;
+  if (lane != 0) return;
   if (b.prio) {
     c->window_limit = next_window_limit(c, b, r, c->window_limit);
     reset_next_min(c, (r + 2) % 3);
   }
   c->round = r + 1;
   c->rounds_executed = r + 1;
-  if (c->list_count[(r + 1) % 3] == 0) {
+  if (!any) {
     c->done = 1;
     c->stop_reason = kStopConverged;
   } else if (b.maximum_rounds && r + 1 >= b.maximum_rounds) {
@@ -112,7 +121,6 @@ __global__ __launch_bounds__(1024) void ordered_advance_kernel(DevBatch b, std::
       c->seg_claim[x * kBarrierStride] = at;
     }
     c->seg_begin[kBarrierGroups] = n;
-    c->list_count[0] = n;
     if (b.instrumentation && n > c->max_list) c->max_list = n;
     if (!first) {
       const std::uint32_t r = c->round;
@@ -136,33 +144,18 @@ __global__ __launch_bounds__(1024) void ordered_advance_kernel(DevBatch b, std::
 // ---------------------------------------------------------------------------
 // Batch preparation.
 // ---------------------------------------------------------------------------
-__global__ void reset_control_kernel(DevControl* c, std::uint32_t window) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    c->window_limit = window;  // round 0 visits the sources' slots (priority 0)
-    for (std::uint32_t i = 0; i < 3 * kBarrierGroups * kBarrierStride; ++i) c->next_min[i] = kInfBits;
-    for (int i = 0; i < 3; ++i) {
-      c->list_count[i] = 0;
-      c->claim[i] = 0;
-    }
-    c->round = 0;
-    c->done = 0;
-    c->stop_reason = kStopNone;
-    c->error_bits = 0;
-    c->barrier_count = 0;
-    c->barrier_generation = 0;
-    c->rounds_executed = 0;
-    c->items_processed = 0;
-    c->edges_examined = 0;
-    c->atomic_attempts = 0;
-    c->atomic_successes = 0;
-    c->max_list = 0;
-    c->edges_relaxed = 0;
-    c->algorithmic_bytes = 0;
-    c->closure_sweeps = 0;
-    c->candidates = 0;
-    for (int p = 0; p < kPhaseCount; ++p) c->phase_cycles[p] = 0;
-    for (std::uint32_t i = 0; i < kMaxArrivalGroups * kBarrierStride; ++i) c->group_arrivals[i] = 0;
-  }
+// One workgroup.
+__global__ __launch_bounds__(1024) void reset_control_kernel(DevControl* c, std::uint32_t* queue,
+                                                             std::uint32_t window) {
+  std::uint32_t* words = reinterpret_cast<std::uint32_t*>(c);
+  for (std::uint32_t i = threadIdx.x; i < sizeof(DevControl) / 4; i += blockDim.x) words[i] = 0;
+  if (queue)
+    for (std::uint32_t i = threadIdx.x; i < kQueueWords / kBarrierStride; i += blockDim.x)
+      queue[i * kBarrierStride] = 0;
+  __syncthreads();
+  for (std::uint32_t i = threadIdx.x; i < 3 * kBarrierGroups * kBarrierStride; i += blockDim.x)
+    c->next_min[i] = kInfBits;
+  if (threadIdx.x == 0) c->window_limit = window;  // round 0 visits the sources' slots (priority 0)
 }
 
 __global__ void fill_u32_kernel(std::uint32_t* p, unsigned long long n, std::uint32_t v) {
@@ -259,7 +252,7 @@ hipError_t relax_launch(std::uint32_t block, bool persistent, bool cooperative,
   if (b.ordered)
     hipLaunchKernelGGL(ordered_advance_kernel, dim3(1), dim3(1024), 0, stream, b, 0u);
   else
-    hipLaunchKernelGGL(relax_advance_kernel, dim3(1), dim3(1), 0, stream, b);
+    hipLaunchKernelGGL(relax_advance_kernel, dim3(1), dim3(64), 0, stream, b);
   return hipGetLastError();
 }
 
@@ -320,7 +313,7 @@ hipError_t coresident_per_cu(int device, int promised, std::uint32_t cus, std::s
   probe.probe = 1;
   int per_cu = promised;
   for (; per_cu >= 1; --per_cu) {
-    hipLaunchKernelGGL(reset_control_kernel, dim3(1), dim3(64), 0, stream, b.control, 0u);
+    hipLaunchKernelGGL(reset_control_kernel, dim3(1), dim3(1024), 0, stream, b.control, nullptr, 0u);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
       e = relax_launch(block, true, true, static_cast<std::uint32_t>(per_cu) * cus, lds_bytes, max_v,
@@ -341,7 +334,7 @@ hipError_t coresident_per_cu(int device, int promised, std::uint32_t cus, std::s
 
 hipError_t prep_launch(const DevGraph& g, const DevBatch& b, std::uint64_t pool_words,
                        hipStream_t stream, bool structure) {
-  hipLaunchKernelGGL(reset_control_kernel, dim3(1), dim3(64), 0, stream, b.control, b.window);
+  hipLaunchKernelGGL(reset_control_kernel, dim3(1), dim3(1024), 0, stream, b.control, b.queue, b.window);
   const std::uint32_t fill_grid = 4096;
   hipLaunchKernelGGL(fill_u32_kernel, dim3(fill_grid), dim3(256), 0, stream, b.dist,
                      static_cast<unsigned long long>(pool_words), kInfBits);

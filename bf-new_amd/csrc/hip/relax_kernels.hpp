@@ -81,6 +81,16 @@ __device__ __forceinline__ Lds carve(std::uint32_t* base, std::uint32_t max_v,
 constexpr int kPushChunk = 6;
 static_assert(kPushChunk % 2 == 0, "boundary records are loaded in pairs");
 
+// Query q changed in round r, and whether it has work queued for r + 1.
+// Every writer of a round stores the same value and later rounds store a
+// larger one, so plain stores suffice (an atomic per visit would queue on
+// the query's line).
+__device__ __forceinline__ void mark_changed(const DevBatch& b, std::uint32_t q, std::uint32_t r,
+                                             bool queued) {
+  b.last_change[q] = r + 1;
+  if (b.pending && queued) b.pending[q] = r + 2;
+}
+
 // Edge records in registers: thread t holds records t, t + B, t + 2B, ... of
 // the range it loaded.
 template <int B, int N>
@@ -163,18 +173,14 @@ __device__ __forceinline__ void visit_pull(const DevGraph& g, const DevBatch& b,
   const std::uint32_t e1 = d.e1;
   const std::uint32_t ei = d.ei;
   const bool resident = ei - e0 <= static_cast<std::uint32_t>(B * EPT);
-  // The internal records are requested first and travel with the table reads
-  // and the slabs; they stay in registers through the tile closure when they
-  // fit (resident), and are not kept across visits.
-  RecordRegs<B, EPT> internal;
-  if (resident) load_records<B, EPT>(internal, g.csc_rec, e0, ei);
-
   // Neighbour k's slab: LDS offset, size and pool offset of its read column,
   // looked up by thread k.  A visit is bound by the latency of its dependent
   // reads, so the table reads of all slabs travel together (two round trips
   // for the list).  Setup of a visit on 256-vertex tiles: 40.1k -> 9.6k
   // cycles; relaxation of 64 queries on 64x64x256 tiles (block Jacobi) 2928
   // -> 2298 us, of 32 point-Jacobi queries on 32x32x128 736 -> 580 us.
+  // (Four rows in flight, or the internal records requested before the
+  // slabs, take 12 to 26 more registers and measured 2 and 5 % slower.)
   for (std::uint32_t k = tid; k < K; k += B) {
     const std::uint32_t nt = g.in_nbr_tiles[nb0 + k];
     const std::uint32_t ns = b.slot_in[in_base + k];
@@ -191,9 +197,9 @@ __device__ __forceinline__ void visit_pull(const DevGraph& g, const DevBatch& b,
   }
   __syncthreads();
   // Stage the read column of every in-neighbour slab (k = 0 is T itself).  A
-  // wave takes four slabs at a time and keeps four 64-word rows of each in
+  // wave takes four slabs at a time and keeps two 64-word rows of each in
   // flight, so a list of up to 16 small slabs costs one round trip.
-  constexpr std::uint32_t kSlabs = 4, kRows = 4, kWaves = B / 64;
+  constexpr std::uint32_t kSlabs = 4, kRows = 2, kWaves = B / 64;
   const std::uint32_t lane = tid & 63u, wave = tid >> 6;
   for (std::uint32_t k0 = wave; k0 < K; k0 += kSlabs * kWaves) {
     const std::uint32_t* src[kSlabs];
@@ -245,11 +251,14 @@ __device__ __forceinline__ void visit_pull(const DevGraph& g, const DevBatch& b,
     const std::uint32_t cb = as_bits(as_float(l.work[l.slots[pk_k(p)] + pk_src(p)]) + w);
     if (cb < l.own[pk_dst(p)]) atomicMin(&l.own[pk_dst(p)], cb);
   };
-  // The first boundary chunk is requested before the internal records are
-  // relaxed, and every later one before its predecessor.
+  // The internal records stay in registers through the tile closure when
+  // they fit (resident), and are not kept across visits.  The first boundary
+  // chunk travels with them.
   constexpr int kStream = stream_records(B);
+  RecordRegs<B, EPT> internal;
   RecordRegs<B, kStream> chunk;
   load_records<B, kStream>(chunk, g.csc_rec, ei, e1);
+  if (resident) load_records<B, EPT>(internal, g.csc_rec, e0, ei);
   for (std::uint32_t base = e0; base < ei; base += B * EPT) {
     if (!resident) load_records<B, EPT>(internal, g.csc_rec, base, ei);
 #pragma unroll
@@ -258,12 +267,10 @@ __device__ __forceinline__ void visit_pull(const DevGraph& g, const DevBatch& b,
   }
   st.mark(1);
   for (std::uint32_t base = ei; base < e1; base += B * kStream) {
-    RecordRegs<B, kStream> next;
-    load_records<B, kStream>(next, g.csc_rec, base + B * kStream, e1);
+    if (base != ei) load_records<B, kStream>(chunk, g.csc_rec, base, e1);
 #pragma unroll
     for (int j = 0; j < kStream; ++j)
       if (chunk.pack[j] != kNone) relax_staged(chunk.pack[j], chunk.w[j]);
-    chunk = next;
   }
   __syncthreads();
   st.mark(3);
@@ -300,13 +307,12 @@ __device__ __forceinline__ void visit_pull(const DevGraph& g, const DevBatch& b,
     changed |= (v != l.work[i]);
   }
   if (__syncthreads_or(changed)) {
-    if (tid == 0) atomic_max_agent(&b.last_change[q], r + 1);
+    if (tid == 0) mark_changed(b, q, r, true);
     // every selected out-neighbour (the tile itself first) reads the new
     // column next round
-    for (std::uint32_t j0 = 0; j0 < d.out_count; j0 += B) {
-      const std::uint32_t j = j0 + tid;
-      const std::uint32_t ns = j < d.out_count ? b.slot_out[d.out_base + j] : kNone;
-      enqueue_wave(b, ns == kNone ? 0u : ns, ns != kNone, r + 1);
+    for (std::uint32_t j = tid; j < d.out_count; j += B) {
+      const std::uint32_t ns = b.slot_out[d.out_base + j];
+      if (ns != kNone) enqueue(b, ns, r + 1);
     }
   }
   st.mark(4);
@@ -574,26 +580,52 @@ __device__ __forceinline__ void visit_push(const DevGraph& g, const DevBatch& b,
   // A marked neighbour holds the smallest candidate pushed into it; with a
   // push window that candidate lowers the neighbour's priority.
   bool marked = false;
-  for (std::uint32_t k0 = 1; k0 < KO; k0 += B) {
-    const std::uint32_t k = k0 + tid;
-    const std::uint32_t low = k < KO ? l.marks[k] : kInfBits;
-    const bool want = low != kInfBits;
-    marked |= want;
-    if (want && b.prio) {
+  for (std::uint32_t k = 1 + tid; k < KO; k += B) {
+    const std::uint32_t low = l.marks[k];
+    if (low == kInfBits) continue;
+    marked = true;
+    if (b.prio) {
       atomic_min_agent(&b.prio[l.slots[k]], low);
       queued_min = min(queued_min, low);
     }
-    enqueue_wave(b, want ? l.slots[k] : 0u, want, r + 1);
+    enqueue(b, l.slots[k], r + 1);
   }
-  if (__syncthreads_or(marked) || pushed_any) {
-    if (tid == 0) atomic_max_agent(&b.last_change[q], r + 1);
-  }
+  const bool queued_any = __syncthreads_or(marked);
+  if (tid == 0 && (queued_any || pushed_any)) mark_changed(b, q, r, queued_any);
   st.mark(4);
 }
 
 // ---------------------------------------------------------------------------
 // Round processing shared by the persistent and host-polled kernels.
 // ---------------------------------------------------------------------------
+// Round r's work list as wave 0 sees it: lane x holds the end of class x's
+// entries in the round's flat order (class 0's entries first).  Wave 0 reads
+// the 64 counts in one step; n is their total.
+struct RoundQueue {
+  std::uint32_t end;
+  std::uint32_t n;
+};
+__device__ __forceinline__ RoundQueue load_round_queue(const DevBatch& b, std::uint32_t r) {
+  const std::uint32_t lane = threadIdx.x & 63u;
+  RoundQueue q;
+  q.end = load_agent(list_count(b, r % 3, lane));
+#pragma unroll
+  for (std::uint32_t off = 1; off < 64; off <<= 1) {
+    const std::uint32_t below = __shfl(q.end, static_cast<int>((lane - off) & 63u));
+    if (lane >= off) q.end += below;
+  }
+  q.n = __shfl(q.end, 63);
+  return q;
+}
+// Slot of flat position i < n (wave 0, i uniform).
+__device__ __forceinline__ std::uint32_t queued_slot(const DevBatch& b, const RoundQueue& q,
+                                                     std::uint32_t li, std::uint32_t i) {
+  const std::uint32_t x = static_cast<std::uint32_t>(__popcll(__ballot(q.end <= i)));
+  const std::uint32_t first = __shfl(q.end, static_cast<int>((x - 1u) & 63u));
+  return b.lists[static_cast<std::size_t>(li) * b.slot_count + class_begin(b.slot_count, x) + i -
+                 (x ? first : 0u)];
+}
+
 // Round r's share of one workgroup.  With a push window (b.prio set), a
 // push slot whose priority is above `limit` is not visited: it keeps its
 // priority and is queued again for round r + 1.  The smallest priority the
@@ -601,7 +633,7 @@ __device__ __forceinline__ void visit_push(const DevGraph& g, const DevBatch& b,
 // next_min counter of its XCD group.
 template <int B, int EPT, bool I, int M>
 __device__ __forceinline__ void process_round(const DevGraph& g, const DevBatch& b, std::uint32_t r,
-                              std::uint32_t n, std::uint32_t limit, const Lds& l) {
+                              const RoundQueue& queue, std::uint32_t limit, const Lds& l) {
   const std::uint32_t chunk = b.items_per_claim ? b.items_per_claim : 1u;
   VisitStats<I> st;
   std::uint32_t queued_min = kInfBits;
@@ -635,8 +667,6 @@ __device__ __forceinline__ void process_round(const DevGraph& g, const DevBatch&
     }
     if (run) ++st.items;
     __syncthreads();
-    // the visit's own enqueues are issued before its item is retired
-    if (b.pending && threadIdx.x == 0) atomic_add_agent(&b.pending[d.query], 0xFFFFFFFFu);
   };
   if (b.ordered) {
     // Slot order: the round's list is cut into one segment per XCD group;
@@ -683,21 +713,46 @@ __device__ __forceinline__ void process_round(const DevGraph& g, const DevBatch&
       for (std::uint32_t i = start; i < end; ++i) visit(b.lists[i]);
     }
   } else {
+    // Chunks of the list are dealt to 64 groups of workgroups (blockIdx % 64)
+    // in turn.  A workgroup's first chunk is its own index, with no claim;
+    // chunks beyond the grid are claimed on the group's counter.  Wave 0
+    // walks the list and hands each slot to the workgroup.  Measured with the
+    // list classes (kQueueClasses) against one claim and one append counter,
+    // relaxation per batch: 32 point-Jacobi lanes on 32x32x128 580 -> 270 us,
+    // 64 queries on 64x64x256 block Jacobi 2298 -> 1722 us and frontier push
+    // 1240 -> 946 us, 256 queries on 128x128x512 15.1 -> 13.8 ms.
     const std::uint32_t li = r % 3;
-    // The first ceil(n / chunk) workgroups claim until the list is exhausted;
-    // the others would only find it exhausted, and skip the claim counter
-    // (in a small round most of the grid would otherwise queue atomics on
-    // its one line).
-    const bool claims = static_cast<unsigned long long>(blockIdx.x) * chunk < n;
-    for (; claims;) {
-      if (threadIdx.x == 0) l.flags[0] = atomic_add_agent(&b.control->claim[li], chunk);
+    const std::uint32_t groups = min(gridDim.x, kQueueClasses);
+    const std::uint32_t group = blockIdx.x % groups;
+    const std::uint32_t dealt = group + groups * ((gridDim.x - group + groups - 1u) / groups);
+    // Position of unit u's first item, kNone when it is past the list.
+    auto begin = [&](unsigned long long u) {
+      const unsigned long long at = u * chunk;
+      return at < queue.n ? static_cast<std::uint32_t>(at) : kNone;
+    };
+    std::uint32_t i = begin(blockIdx.x);
+    std::uint32_t left = chunk;
+    for (;;) {
+      if (threadIdx.x < 64) {
+        if (left == 0) {
+          i = begin(dealt);
+          if (i != kNone) {
+            std::uint32_t t = 0;
+            if (threadIdx.x == 0) t = atomic_add_agent(list_claim(b, li, group), 1u);
+            t = __builtin_amdgcn_readfirstlane(__shfl(t, 0));
+            i = begin(dealt + static_cast<unsigned long long>(groups) * t);
+          }
+          left = chunk;
+        }
+        const std::uint32_t s = i < queue.n ? queued_slot(b, queue, li, i) : kNone;
+        if (threadIdx.x == 0) l.flags[0] = s;
+        i += i != kNone;
+        --left;
+      }
       __syncthreads();
-      const std::uint32_t start = l.flags[0];
-      __syncthreads();
-      if (start >= n) break;
-      const std::uint32_t end = min(start + chunk, n);
-      for (std::uint32_t i = start; i < end; ++i)
-        visit(b.lists[static_cast<std::size_t>(li) * b.slot_count + i]);
+      const std::uint32_t s = l.flags[0];
+      if (s == kNone) break;
+      visit(s);
     }
   }
   if (b.prio) {
@@ -745,16 +800,24 @@ __global__ __launch_bounds__(B, MW) void relax_persistent_kernel(DevGraph g, Dev
   std::uint32_t n = 0;
   std::uint32_t limit = b.prio ? load_agent(&c->window_limit) : 0u;
   for (;;) {
-    n = load_agent(&c->list_count[r % 3]);
-    if (n == 0 || (b.maximum_rounds && r >= b.maximum_rounds)) break;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-      store_agent(&c->list_count[(r + 2) % 3], 0u);
-      store_agent(&c->claim[(r + 2) % 3], 0u);
-      // read after the barrier of round r - 2, written in round r + 1
-      if (b.prio) reset_next_min(c, (r + 2) % 3);
-      if (b.instrumentation) atomicMax(&c->max_list, static_cast<unsigned long long>(n));
+    RoundQueue queue{};
+    if (threadIdx.x < 64) {
+      queue = load_round_queue(b, r);
+      if (threadIdx.x == 0) l.flags[5] = queue.n;
     }
-    process_round<B, EPT, I, M>(g, b, r, n, limit, l);
+    __syncthreads();
+    n = l.flags[5];
+    if (n == 0 || (b.maximum_rounds && r >= b.maximum_rounds)) break;
+    if (blockIdx.x == 0 && threadIdx.x < kQueueClasses) {
+      store_agent(list_count(b, (r + 2) % 3, threadIdx.x), 0u);
+      store_agent(list_claim(b, (r + 2) % 3, threadIdx.x), 0u);
+      if (threadIdx.x == 0) {
+        // read after the barrier of round r - 2, written in round r + 1
+        if (b.prio) reset_next_min(c, (r + 2) % 3);
+        if (b.instrumentation) atomicMax(&c->max_list, static_cast<unsigned long long>(n));
+      }
+    }
+    process_round<B, EPT, I, M>(g, b, r, queue, limit, l);
     if (!grid_barrier_grouped(c, gridDim.x)) return;  // error bits set; the host reports a device failure
     if (b.prio) limit = next_window_limit(c, b, r, limit);
     ++r;
@@ -779,9 +842,10 @@ __global__ __launch_bounds__(B, MW) void relax_round_kernel(DevGraph g, DevBatch
   DevControl* c = b.control;
   if (load_agent(&c->done)) return;
   const std::uint32_t r = load_agent(&c->round);
-  const std::uint32_t n = b.ordered ? 0u : load_agent(&c->list_count[r % 3]);
+  RoundQueue queue{};
+  if (!b.ordered && threadIdx.x < 64) queue = load_round_queue(b, r);
   const std::uint32_t limit = b.prio ? load_agent(&c->window_limit) : 0u;
-  process_round<B, EPT, I, M>(g, b, r, n, limit, l);
+  process_round<B, EPT, I, M>(g, b, r, queue, limit, l);
 }
 
 // ---------------------------------------------------------------------------

@@ -12,7 +12,7 @@
 //   relax    -- rounds_per_chunk rounds of the shared round kernel over every
 //               admitted query: queries admitted now run alongside queries
 //               that are half way;
-//   harvest  -- a query whose queued-work counter reached zero has converged;
+//   harvest  -- a query with no work queued for the next round has converged;
 //               its target label (and path length) is copied out, its slots
 //               return to the arena and a response is posted.
 // Requests therefore join the running batch between chunks, and their work
@@ -108,6 +108,7 @@ __global__ void admit_kernel(DevGraph g, DevBatch b, const AdmitRecord* records,
     const bool jacobi = r.engine == kJacobiPull;
     if (jacobi) column[npt + (u - v0)] = 0u;
     enqueue(b, s, round);
+    b.pending[q] = round + 1;
     if (jacobi) {
       const std::uint32_t KO = g.out_nbr_offsets[T + 1] - g.out_nbr_offsets[T];
       for (std::uint32_t k = 0; k < KO; ++k) {
@@ -119,13 +120,13 @@ __global__ void admit_kernel(DevGraph g, DevBatch b, const AdmitRecord* records,
   }
 }
 
-// Reports converged queries: pending work reached zero.
+// Reports converged queries: those with no work queued for the next round.
 __global__ void harvest_kernel(DevGraph g, DevBatch b, std::uint32_t capacity,
                                std::uint32_t* active, std::uint32_t* done_list,
                                std::uint32_t* result_bits) {
   const std::uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= capacity || !active[q]) return;
-  if (load_agent(&b.pending[q]) != 0) return;
+  if (b.pending[q] > b.control->round) return;
   active[q] = 0;
   const std::uint32_t pos = atomicAdd(&done_list[0], 1u);
   done_list[1 + pos] = q;
@@ -162,12 +163,9 @@ __global__ void server_init_kernel(DevBatch b, std::uint32_t capacity, std::uint
     const_cast<std::uint32_t*>(b.slot_out_base)[i] = i * kout;
     b.stamp[i] = 0;
   }
+  if (i < kQueueWords / kBarrierStride) b.queue[i * kBarrierStride] = 0;
   if (i == 0) {
     DevControl* c = b.control;
-    for (int k = 0; k < 3; ++k) {
-      c->list_count[k] = 0;
-      c->claim[k] = 0;
-    }
     c->round = 0;
     c->done = 1;
     c->stop_reason = 0;
@@ -229,7 +227,7 @@ struct bfn_server_s {
                 *d_src = nullptr, *d_tgt_off = nullptr, *d_tgt = nullptr, *d_engine = nullptr,
                 *d_last = nullptr, *d_pending = nullptr, *d_active = nullptr, *d_done = nullptr,
                 *d_result = nullptr, *d_clean = nullptr, *d_summary = nullptr,
-                *d_upload_tiles = nullptr;
+                *d_upload_tiles = nullptr, *d_queue = nullptr;
   unsigned long long *d_slot_dist = nullptr, *d_frame_base = nullptr, *d_lengths = nullptr,
                      *d_path_offsets = nullptr;
   // Compact-path arenas of one step's converged queries (grown on demand).
@@ -562,7 +560,7 @@ int32_t bfn_server_create(bfn_device device, bfn_graph graph, const bfn_server_o
             alloc(&sv->d_result, 4 * Q) && alloc(&sv->d_clean, 4 * Q) &&
             alloc(&sv->d_summary, 28 * Q) && alloc(&sv->d_lengths, 8 * Q) &&
             alloc(&sv->d_frame_base, 8 * Q) && alloc(&sv->d_path_offsets, 8 * Q) &&
-            alloc(&sv->d_control, sizeof(DevControl)) &&
+            alloc(&sv->d_control, sizeof(DevControl)) && alloc(&sv->d_queue, 4ull * kQueueWords) &&
             alloc(&sv->d_records, sizeof(AdmitRecord) * Q) &&
             alloc(&sv->d_upload_tiles, 4ull * sv->upload_tile_capacity);
   if (!ok) return bail(BFN_E_OUT_OF_MEMORY, "server allocation failed");
@@ -610,8 +608,9 @@ int32_t bfn_server_create(bfn_device device, bfn_graph graph, const bfn_server_o
   b.dist = sv->d_pool;
   b.last_change = sv->d_last;
   b.pending = sv->d_pending;
+  b.queue = sv->d_queue;
   b.control = sv->d_control;
-  const std::uint32_t n = std::max(sv->Scap, sv->Qcap + 1);
+  const std::uint32_t n = std::max({sv->Scap, sv->Qcap + 1, kQueueWords / kBarrierStride});
   hipLaunchKernelGGL(server_init_kernel, dim3((n + 255) / 256), dim3(256), 0, sv->stream, b, sv->Qcap,
                      sv->Scap, sv->slab_words, sv->kin, sv->kout, sv->d_active, sv->d_src_off,
                      sv->d_tgt_off, sv->d_clean);

@@ -131,6 +131,7 @@ inline long long clock64() {
 #define __builtin_amdgcn_fence(o, s) ((void)0)
 #define __builtin_amdgcn_s_sleep(n) emu::yield()
 #define __builtin_amdgcn_readfirstlane(x) (x)
+#define __builtin_amdgcn_s_waitcnt(x) ((void)0)
 
 template <typename T> inline T min(T a, T b) { return b < a ? b : a; }
 template <typename T> inline T max(T a, T b) { return a < b ? b : a; }

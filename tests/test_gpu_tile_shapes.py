@@ -2,7 +2,8 @@
 stages at a time (64-word rows, four rows per slab, the registers that hold a
 tile's internal records), against the oracle bit for bit.  The 9 x 8 grid
 clamps its long edges, so tiles have between 5 and 13 neighbours, and the
-boxes leave some of them out."""
+boxes leave some of them out; the batches have fewer slots than work-list
+classes and more, and claims of several items."""
 import numpy as np
 import pytest
 
@@ -16,7 +17,8 @@ CONFIGS = [
     dict(engine=bfn.JACOBI_PULL, control=bfn.CHUNKED, sweeps=0, boundary=0),
     dict(engine=bfn.DENSE_CHAOTIC_PUSH, control=bfn.PER_ROUND, sweeps=0, boundary=0),
     dict(engine=bfn.FRONTIER_PUSH, control=bfn.PERSISTENT, sweeps=0, boundary=0),
-    dict(engine=bfn.FRONTIER_PUSH, control=bfn.CHUNKED, sweeps=0, boundary=1, window=4.0),
+    dict(engine=bfn.FRONTIER_PUSH, control=bfn.CHUNKED, sweeps=0, boundary=1, window=4.0,
+         per_claim=5),
 ]
 
 
@@ -37,7 +39,8 @@ def test_tile_shapes_bit_exact(device, nodes, block):
         ws.submit(dg, batch, bfn.run_options(engine=c["engine"], control_mode=c["control"],
                                              rounds_per_chunk=3, block_size=block),
                   bfn.tuning(tile_sweeps=c["sweeps"], boundary_mode=c["boundary"],
-                             push_window=c.get("window", 0.0)))
+                             push_window=c.get("window", 0.0),
+                             items_per_claim=c.get("per_claim", 1)))
         assert ws.status()[0].converged == 1, c
         for i in range(len(qs)):
             assert np.array_equal(bits(ws.distances(i)), bits(want[i])), (c, i)
