@@ -65,11 +65,20 @@ constexpr std::uint32_t kLdsFlagWords = 16;
 // holds the push visit (or only the pull visit) needs fewer registers per
 // lane than one that holds both, so more waves are resident.
 constexpr std::uint32_t kEnginesMixed = 0;
-constexpr std::uint32_t kEnginesPush = 1;
+constexpr std::uint32_t kEnginesPush = 1;      // boundary_mode 1
 constexpr std::uint32_t kEnginesPull = 2;
 // Workgroups are dispatched round-robin over the 8 XCDs (blockIdx % 8):
 // per-XCD counters (claims, window minima) are indexed by that group.  The
 // grid barrier gathers its arrivals on kArrivalGroups counters (a multiple
+constexpr std::uint32_t kEnginesPushLds = 3;   // boundary_mode 0
+__host__ __device__ constexpr bool holds_pull(std::uint32_t engines) {
+  return engines == kEnginesMixed || engines == kEnginesPull;
+}
+__host__ __device__ constexpr bool holds_push(std::uint32_t engines) { return engines != kEnginesPull; }
+inline std::uint32_t engine_set(bool any_jacobi, bool any_push, bool proposals) {
+  if (any_jacobi) return any_push ? kEnginesMixed : kEnginesPull;
+  return proposals ? kEnginesPushLds : kEnginesPush;
+}
 // of 8, so each counter's workgroups share an XCD) before the top counter.
 constexpr std::uint32_t kBarrierGroups = 8;
 constexpr std::uint32_t kMaxArrivalGroups = 64;  // arrival counters in DevControl
@@ -211,7 +220,7 @@ struct DevBatch {
   std::uint32_t min_waves;        // kernel variant bounded to >= this many waves per SIMD
   std::uint32_t ordered;          // slot-order claims: queue as bits in `active`
   std::uint32_t window;           // push window (float bits), 0 = off
-  std::uint32_t engines;          // kEnginesMixed / kEnginesPush / kEnginesPull: the
+  std::uint32_t engines;          // one of kEngines*: the
                                   // relaxation kernel variant, by the engines the batch holds
   std::uint32_t probe;            // persistent kernel: pass one grid barrier and exit
   const std::uint32_t* tile_begin;      // [Q]   first position of q in query_tiles

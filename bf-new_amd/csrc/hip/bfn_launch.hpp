@@ -44,7 +44,7 @@ hipError_t relax_occupancy(std::uint32_t engines, std::uint32_t block, bool pers
                            bool instrumented, std::uint32_t min_waves, std::size_t lds_bytes,
                            int* blocks_per_cu);
 // The kernel variants of one engine set (relax_mixed.hip, relax_push.hip,
-// relax_pull.hip); relax_launch and relax_occupancy pick by engine set.
+// relax_push_lds.hip, relax_pull.hip); relax_launch and relax_occupancy pick by engine set.
 #define BFN_RELAX_ENGINE_SET(name)                                                             \
   hipError_t relax_launch_##name(std::uint32_t block, bool persistent, bool cooperative,      \
                                  std::uint32_t grid, std::size_t lds_bytes, std::uint32_t max_v, \
@@ -55,6 +55,7 @@ hipError_t relax_occupancy(std::uint32_t engines, std::uint32_t block, bool pers
                                     int* blocks_per_cu);
 BFN_RELAX_ENGINE_SET(mixed)
 BFN_RELAX_ENGINE_SET(push)
+BFN_RELAX_ENGINE_SET(push_lds)
 BFN_RELAX_ENGINE_SET(pull)
 #undef BFN_RELAX_ENGINE_SET
 // Resets the control block, fills the labels and seeds round 0; with

@@ -1065,7 +1065,7 @@ int32_t bfn_batch_submit(bfn_workspace ws, bfn_graph graph, const bfn_batch_desc
                                              std::to_string(lds_bytes) + " > " +
                                              std::to_string(lds_limit) + " bytes)");
   int per_cu = 0;
-  const std::uint32_t engines = !p.any_jacobi ? kEnginesPush : !p.any_push ? kEnginesPull : kEnginesMixed;
+  const std::uint32_t engines = engine_set(p.any_jacobi, p.any_push, proposals);
   BFN_HIP(relax_occupancy(engines, o->block_size, o->control_mode == 0, o->instrumentation != 0,
                           t.min_waves, lds_bytes, &per_cu));
   if (per_cu <= 0) return fail(BFN_E_NOT_REPRESENTABLE, "relaxation kernel cannot be resident");

@@ -240,7 +240,7 @@ int32_t bfn_batch_run_static(bfn_graph graph, const bfn_batch_desc* d, const bfn
   const bool persistent = o->control_mode == 0;
   int per_cu = 0;
   BFN_HIP_STATIC(hipSetDevice(gh.ordinal));
-  const std::uint32_t engines = !any_jacobi ? kEnginesPush : !any_push ? kEnginesPull : kEnginesMixed;
+  const std::uint32_t engines = engine_set(any_jacobi, any_push, false);
   BFN_HIP_STATIC(relax_occupancy(engines, o->block_size, persistent, o->instrumentation != 0, t.min_waves,
                                  lds_bytes, &per_cu));
   if (per_cu <= 0) return fail(BFN_E_NOT_REPRESENTABLE, "relaxation kernel cannot be resident");

@@ -2,7 +2,7 @@
 // between round launches, batch preparation (control reset, label fill,
 // slot tables, seeds) and the launch dispatch to the kernel variant of a
 // batch's engine set (relax_kernels.hpp, instantiated by relax_mixed.hip,
-// relax_push.hip and relax_pull.hip).
+// relax_push.hip, relax_push_lds.hip and relax_pull.hip).
 #include "bfn_launch.hpp"
 
 #include <mutex>
@@ -193,7 +193,7 @@ __global__ void prep_slots_kernel(DevGraph g, DevBatch b, std::uint32_t structur
   if (b.prio) b.prio[s] = kInfBits;
   // the relaxation kernel variant must hold the engine of every slot
   const bool pull = b.engine[q] == kJacobiPull;
-  if ((b.engines == kEnginesPush && pull) || (b.engines == kEnginesPull && !pull))
+  if (pull ? !holds_pull(b.engines) : !holds_push(b.engines))
     atomicOr(&b.control->error_bits, 4u);
   b.last_change[q] = 0;
   if (structure && b.slot_desc) const_cast<SlotDesc*>(b.slot_desc)[s] = make_slot_desc(g, b, s);
@@ -242,6 +242,9 @@ hipError_t relax_launch(std::uint32_t block, bool persistent, bool cooperative,
     case kEnginesPush:
       e = relax_launch_push(block, persistent, cooperative, grid, lds_bytes, max_v, work_words, g, b, stream);
       break;
+    case kEnginesPushLds:
+      e = relax_launch_push_lds(block, persistent, cooperative, grid, lds_bytes, max_v, work_words, g, b, stream);
+      break;
     case kEnginesPull:
       e = relax_launch_pull(block, persistent, cooperative, grid, lds_bytes, max_v, work_words, g, b, stream);
       break;
@@ -262,6 +265,8 @@ hipError_t relax_occupancy(std::uint32_t engines, std::uint32_t block, bool pers
   switch (engines) {
     case kEnginesPush:
       return relax_occupancy_push(block, persistent, instrumented, min_waves, lds_bytes, blocks_per_cu);
+    case kEnginesPushLds:
+      return relax_occupancy_push_lds(block, persistent, instrumented, min_waves, lds_bytes, blocks_per_cu);
     case kEnginesPull:
       return relax_occupancy_pull(block, persistent, instrumented, min_waves, lds_bytes, blocks_per_cu);
     default:

@@ -1,4 +1,5 @@
-// relax_push.hip -- the relaxation kernel variants for batches of push queries only (dense chaotic and frontier push).
+// relax_push.hip -- the relaxation kernel variants for batches of push queries only (dense chaotic and frontier push)
+// whose boundary candidates go straight to the neighbours' labels (boundary_mode 1).
 #include "relax_kernels.hpp"
 
 #include "bfn_launch.hpp"
