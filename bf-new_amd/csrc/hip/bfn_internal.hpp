@@ -63,13 +63,13 @@ constexpr std::uint32_t kLdsFlagWords = 16;
 
 // Relaxation kernel variants by the engines of a batch: a kernel that only
 // holds the push visit (or only the pull visit) needs fewer registers per
-// lane than one that holds both, so more waves are resident.
+// lane than one that holds both, so more waves are resident.  The push visit
+// comes with direct boundary pushes only, and with LDS proposals only (in one
+// kernel the proposals cost the direct visits registers: 256 queries on
+// 128x128x512, 13.8 -> 14.3 ms).
 constexpr std::uint32_t kEnginesMixed = 0;
 constexpr std::uint32_t kEnginesPush = 1;      // boundary_mode 1
 constexpr std::uint32_t kEnginesPull = 2;
-// Workgroups are dispatched round-robin over the 8 XCDs (blockIdx % 8):
-// per-XCD counters (claims, window minima) are indexed by that group.  The
-// grid barrier gathers its arrivals on kArrivalGroups counters (a multiple
 constexpr std::uint32_t kEnginesPushLds = 3;   // boundary_mode 0
 __host__ __device__ constexpr bool holds_pull(std::uint32_t engines) {
   return engines == kEnginesMixed || engines == kEnginesPull;
@@ -79,6 +79,9 @@ inline std::uint32_t engine_set(bool any_jacobi, bool any_push, bool proposals) 
   if (any_jacobi) return any_push ? kEnginesMixed : kEnginesPull;
   return proposals ? kEnginesPushLds : kEnginesPush;
 }
+// Workgroups are dispatched round-robin over the 8 XCDs (blockIdx % 8):
+// per-XCD counters (claims, window minima) are indexed by that group.  The
+// grid barrier gathers its arrivals on kArrivalGroups counters (a multiple
 // of 8, so each counter's workgroups share an XCD) before the top counter.
 constexpr std::uint32_t kBarrierGroups = 8;
 constexpr std::uint32_t kMaxArrivalGroups = 64;  // arrival counters in DevControl
@@ -269,6 +272,12 @@ struct QueryStatusDev {
   std::uint32_t engine;
 };
 
+// Bits of PathArgs::query_clean: the query converged without error; pass 1
+// walked one of its targets with backtracking (its frames hold only the last
+// walk, so pass 2 walks again).
+constexpr std::uint32_t kPathClean = 1u;
+constexpr std::uint32_t kPathGeneral = 2u;
+
 // Arguments of the compact-path passes.
 struct PathArgs {
   DevGraph g;
@@ -277,18 +286,25 @@ struct PathArgs {
   std::uint32_t pass;                   // 1: summaries + lengths, 2: emit arenas
   std::uint32_t target_total;
   std::uint32_t stamp_base;             // target t's walk marks onpath with stamp_base + t + 1
-  const std::uint32_t* query_clean;     // [Q] converged without error
+  std::uint32_t* query_clean;           // [Q] kPath* bits
   const unsigned long long* frame_base; // [Q] frame scratch offset
+  unsigned long long frame_words;       // frames of the whole batch
+  std::uint32_t frame_slab;             // frames per selected tile, or 0: up to the next query's base
+  std::uint32_t most_targets;           // largest target count of a query
   std::uint32_t* frame_vertex;
-  std::uint32_t* frame_last;
+  std::uint32_t* frame_last;            // EdgeId last tried (backtracking) / label (descending)
   std::uint32_t* frame_via;
   std::uint32_t* onpath;                // pool-sized stamps
   std::uint32_t* summaries;             // [targets][7]
   unsigned long long* lengths;          // [targets] vertex count of each path
   const unsigned long long* offsets;    // [targets+1] (pass 2)
+  unsigned long long arena_capacity;    // pass 2 writes nothing when the paths need more
   std::uint32_t* arena_vertices;
   std::uint32_t* arena_labels;
   std::uint32_t* arena_edges;
+  std::uint32_t* host_vertices;         // pinned copies of the arenas, or null
+  std::uint32_t* host_labels;
+  std::uint32_t* host_edges;
   const std::uint32_t* query_list;      // queries to reconstruct (null: all)
   std::uint32_t jacobi_copy_from_control;  // take the column from round parity
   std::uint32_t pad2;

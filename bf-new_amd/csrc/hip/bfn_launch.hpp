@@ -139,7 +139,8 @@ hipError_t gather_region_launch(const DevGraph& g, const DevBatch& b, std::uint3
                                 const unsigned long long* offsets, std::uint32_t* out,
                                 hipStream_t stream);
 hipError_t finalize_launch(const DevGraph& g, const DevBatch& b,
-                           const unsigned long long* relaxations, void* out, hipStream_t stream);
+                           const unsigned long long* relaxations, void* out,
+                           std::uint32_t* path_state, hipStream_t stream);
 hipError_t relaxation_count_launch(const DevGraph& g, const DevBatch& b,
                                    unsigned long long* out, hipStream_t stream);
 hipError_t occupancy_launch(const std::uint32_t* arena, unsigned long long n, int* occ,

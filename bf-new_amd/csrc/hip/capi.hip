@@ -162,9 +162,9 @@ struct bfn_workspace_s {
   // batch metadata in one device buffer + separately grown state
   DeviceBuffer meta, slot_in, slot_out, slot_out_off, slot_desc, stamp, prio, lists, pool, last_change, control, queue,
       status, relax,
-      scratch_v, paths_summary, paths_len, paths_off, frames, onpath, clean, arena_v, arena_l,
+      scratch_v, paths_out, paths_len, frames, onpath, clean, arena_v, arena_l,
       arena_e, occupancy, region_off;
-  PinnedBuffer staging, h_status, h_control, h_paths;
+  PinnedBuffer staging, h_status, h_control, h_paths, h_arena;
   // last batch
   bfn_graph graph = nullptr;
   DevBatch view{};
@@ -178,9 +178,11 @@ struct bfn_workspace_s {
   std::size_t lds_bytes = 0;
   const unsigned long long* frame_base_ptr = nullptr;  // in `meta`
   bool submitted = false, completed = false, have_paths = false;
-  bool paths_counted = false;  // pass 1 of this completion's paths is on the host
+  bool paths_counted = false;  // summaries and offsets of this completion's paths are on the host
+  bool paths_emitted = false;  // and the paths themselves in h_arena
   bool slots_resolved = false; // the batch's neighbour slots and descriptors are on the device
-  std::uint64_t arena_vertices = 0;
+  std::uint64_t arena_vertices = 0, arena_room = 0;
+  std::uint32_t most_targets = 0;
   // Path-kernel marks in `onpath`: the next pass marks with stamps
   // [path_stamp + 1, path_stamp + targets]; the buffer was last cleared at
   // onpath_cleared for onpath_cleared_words words.
@@ -879,7 +881,7 @@ int32_t run_resident_batch(bfn_workspace ws) {
   const DevBatch& b = ws->view;
   ws->completed = false;
   ws->have_paths = false;
-  ws->paths_counted = false;
+  ws->paths_counted = ws->paths_emitted = false;
   BFN_HIP(hipEventRecord(ws->ev_start, s));
   const bool graph_mode = t.use_graph && o.control_mode != 0;
   unsigned long long* relax = t.count_relaxations ? ws->relax.as<unsigned long long>() : nullptr;
@@ -889,7 +891,7 @@ int32_t run_resident_batch(bfn_workspace ws) {
       e = fill_launch(reinterpret_cast<std::uint32_t*>(relax), 2ull * b.query_count, 0u, s);
       if (e == hipSuccess) e = relaxation_count_launch(g->view, b, relax, s);
     }
-    if (e == hipSuccess) e = finalize_launch(g->view, b, relax, ws->status.ptr, s);
+    if (e == hipSuccess) e = finalize_launch(g->view, b, relax, ws->status.ptr, ws->clean.as<std::uint32_t>(), s);
     if (e == hipSuccess)
       e = hipMemcpyAsync(ws->h_status.ptr, ws->status.ptr, sizeof(QueryStatusDev) * b.query_count,
                          hipMemcpyDeviceToHost, s);
@@ -1015,7 +1017,8 @@ int32_t bfn_batch_submit(bfn_workspace ws, bfn_graph graph, const bfn_batch_desc
   // From here on the workspace holds no batch until this one is bound: a
   // refused submit never leaves the previous batch's results readable under
   // the new batch's description.
-  ws->submitted = ws->completed = ws->have_paths = ws->paths_counted = false;
+  ws->submitted = ws->completed = ws->have_paths = false;
+  ws->paths_counted = ws->paths_emitted = false;
   ws->slots_resolved = false;
   if (ws->device != graph->device) return fail(BFN_E_INVALID_ARGUMENT, "graph is on another device");
   if (int32_t rc = validate_options(o)) return rc;
@@ -1104,6 +1107,7 @@ int32_t bfn_batch_submit(bfn_workspace ws, bfn_graph graph, const bfn_batch_desc
   BFN_HIP(ws->queue.reserve(4ull * kQueueWords));
   BFN_HIP(ws->status.reserve(sizeof(QueryStatusDev) * Q));
   BFN_HIP(ws->relax.reserve(8ull * Q));
+  BFN_HIP(ws->clean.reserve(4ull * Q));
   BFN_HIP(ws->h_status.reserve(sizeof(QueryStatusDev) * Q));
   BFN_HIP(ws->h_control.reserve(sizeof(DevControl)));
   BFN_HIP(hipMemcpyAsync(ws->meta.ptr, h, meta_bytes, hipMemcpyHostToDevice, ws->stream));
@@ -1116,6 +1120,9 @@ int32_t bfn_batch_submit(bfn_workspace ws, bfn_graph graph, const bfn_batch_desc
   ws->options = *o;
   ws->tuning = t;
   ws->h_target_off.assign(d->target_offsets, d->target_offsets + Q + 1);
+  ws->most_targets = 0;
+  for (std::uint32_t q = 0; q < Q; ++q)
+    ws->most_targets = std::max(ws->most_targets, d->target_offsets[q + 1] - d->target_offsets[q]);
   ws->h_tile_off.assign(d->tile_offsets, d->tile_offsets + Q + 1);
   ws->h_tiles.assign(d->selected_tiles, d->selected_tiles + S);
   ws->h_engine = p.engine;
@@ -1301,14 +1308,13 @@ int32_t bfn_batch_paths(bfn_workspace ws, bfn_target_summary* summaries, uint64_
   hipStream_t s = ws->stream;
   const std::uint32_t NT = ws->h_target_off[ws->Q];
   const DevControl* c = ws->h_control.as<DevControl>();
-  const QueryStatusDev* qs = ws->h_status.as<QueryStatusDev>();
-  BFN_HIP(ws->paths_summary.reserve(28ull * NT));
+  // Summaries and offsets sit in one buffer (one copy to the host).
+  const std::size_t off_at = align_up(28ull * NT, 8), out_bytes = off_at + 8ull * (NT + 1);
+  BFN_HIP(ws->paths_out.reserve(out_bytes));
   BFN_HIP(ws->paths_len.reserve(8ull * NT));
-  BFN_HIP(ws->paths_off.reserve(8ull * (NT + 1)));
   BFN_HIP(ws->frames.reserve(12ull * std::max<std::uint64_t>(ws->frame_words, 1)));
   BFN_HIP(ws->onpath.reserve(4ull * std::max<std::uint64_t>(ws->pool_words, 1)));
-  BFN_HIP(ws->clean.reserve(4ull * ws->Q));
-  BFN_HIP(ws->h_paths.reserve(28ull * NT + 8ull * (NT + 1) + 4ull * ws->Q));
+  BFN_HIP(ws->h_paths.reserve(out_bytes));
   char* hp = ws->h_paths.as<char>();
   PathArgs a{};
   a.g = ws->graph->view;
@@ -1318,13 +1324,16 @@ int32_t bfn_batch_paths(bfn_workspace ws, bfn_target_summary* summaries, uint64_
   a.target_total = NT;
   a.query_clean = ws->clean.as<std::uint32_t>();
   a.frame_base = ws->frame_base_ptr;
+  a.frame_words = ws->frame_words;
+  a.most_targets = ws->most_targets;
   a.frame_vertex = ws->frames.as<std::uint32_t>();
   a.frame_last = a.frame_vertex + ws->frame_words;
   a.frame_via = a.frame_last + ws->frame_words;
   a.onpath = ws->onpath.as<std::uint32_t>();
-  a.summaries = ws->paths_summary.as<std::uint32_t>();
+  a.summaries = ws->paths_out.as<std::uint32_t>();
   a.lengths = ws->paths_len.as<unsigned long long>();
-  a.offsets = ws->paths_off.as<unsigned long long>();
+  unsigned long long* offsets = reinterpret_cast<unsigned long long*>(ws->paths_out.as<char>() + off_at);
+  a.offsets = offsets;
   // Every pass of the path kernel marks the vertices on its walks with its
   // own stamp range, so the marks that earlier passes (and earlier batches)
   // left on found paths never match a later stamp: the marks are cleared
@@ -1343,44 +1352,64 @@ int32_t bfn_batch_paths(bfn_workspace ws, bfn_target_summary* summaries, uint64_
     ws->path_stamp += NT;
     return hipSuccess;
   };
-  // Pass 1 (summaries, lengths, offsets) runs once per completed batch: a
-  // second call, the one that brings the arenas, reuses its results.
+  // Room for `vertices` path vertices on the device and in pinned memory.
+  auto make_room = [&](std::uint64_t vertices) -> hipError_t {
+    if (vertices <= ws->arena_room) return hipSuccess;
+    ws->arena_room = 0;
+    hipError_t e = ws->arena_v.reserve(4ull * vertices);
+    if (e == hipSuccess) e = ws->arena_l.reserve(4ull * vertices);
+    if (e == hipSuccess) e = ws->arena_e.reserve(4ull * vertices);
+    if (e == hipSuccess) e = ws->h_arena.reserve(12ull * vertices);
+    if (e == hipSuccess) ws->arena_room = vertices;
+    return e;
+  };
+  // Pass 2 writes the paths to the device arenas (what occupancy counts) and
+  // to pinned host memory, where a path's few hundred bytes cost less than
+  // three copies.
+  auto emit = [&]() -> hipError_t {
+    hipError_t e = take_stamps();
+    if (e != hipSuccess) return e;
+    a.pass = 2;
+    a.arena_capacity = ws->arena_room;
+    a.arena_vertices = ws->arena_v.as<std::uint32_t>();
+    a.arena_labels = ws->arena_l.as<std::uint32_t>();
+    a.arena_edges = ws->arena_e.as<std::uint32_t>();
+    a.host_vertices = ws->h_arena.as<std::uint32_t>();
+    a.host_labels = a.host_vertices + ws->arena_room;
+    a.host_edges = a.host_labels + ws->arena_room;
+    return paths_launch(a, ws->Q, s);
+  };
+  // Both passes run once per completed batch, pass 2 in the room that earlier
+  // paths had (or 64 vertices per target): the second call, the one that
+  // brings the arenas, finds the paths on the host unless they needed more.
   if (!ws->paths_counted) {
-    std::uint32_t* hclean = reinterpret_cast<std::uint32_t*>(hp + 28ull * NT + 8ull * (NT + 1));
-    for (std::uint32_t q = 0; q < ws->Q; ++q)
-      hclean[q] = (qs[q].converged && qs[q].error_bits == 0) ? 1u : 0u;
-    BFN_HIP(hipMemcpyAsync(ws->clean.ptr, hclean, 4ull * ws->Q, hipMemcpyHostToDevice, s));
+    BFN_HIP(make_room(std::min<std::uint64_t>(64ull * NT, 1ull << 20)));
     BFN_HIP(take_stamps());
     BFN_HIP(paths_launch(a, ws->Q, s));
-    BFN_HIP(scan_u64_launch(a.lengths, ws->paths_off.as<unsigned long long>(), NT, s));
-    BFN_HIP(hipMemcpyAsync(hp, ws->paths_summary.ptr, 28ull * NT, hipMemcpyDeviceToHost, s));
-    BFN_HIP(hipMemcpyAsync(hp + 28ull * NT, ws->paths_off.ptr, 8ull * (NT + 1), hipMemcpyDeviceToHost, s));
+    BFN_HIP(scan_u64_launch(a.lengths, offsets, NT, s));
+    BFN_HIP(emit());
+    BFN_HIP(hipMemcpyAsync(hp, ws->paths_out.ptr, out_bytes, hipMemcpyDeviceToHost, s));
     BFN_HIP(hipStreamSynchronize(s));
     ws->paths_counted = true;
+    ws->paths_emitted = reinterpret_cast<const std::uint64_t*>(hp + off_at)[NT] <= ws->arena_room;
   }
   std::memcpy(summaries, hp, 28ull * NT);
-  std::memcpy(path_offsets, hp + 28ull * NT, 8ull * (NT + 1));
+  std::memcpy(path_offsets, hp + off_at, 8ull * (NT + 1));
   const std::uint64_t total = path_offsets[NT];
   *vertex_total = total;
   if (!vertices && !labels && !edge_ids) return BFN_OK;
   if (!vertices || !labels || !edge_ids) return fail(BFN_E_INVALID_ARGUMENT, "arenas must all be given");
   if (arena_capacity < total) return fail(BFN_E_INVALID_ARGUMENT, "arena capacity too small");
-  BFN_HIP(ws->arena_v.reserve(4ull * std::max<std::uint64_t>(total, 1)));
-  BFN_HIP(ws->arena_l.reserve(4ull * std::max<std::uint64_t>(total, 1)));
-  BFN_HIP(ws->arena_e.reserve(4ull * std::max<std::uint64_t>(total, 1)));
-  BFN_HIP(take_stamps());
-  a.pass = 2;
-  a.arena_vertices = ws->arena_v.as<std::uint32_t>();
-  a.arena_labels = ws->arena_l.as<std::uint32_t>();
-  a.arena_edges = ws->arena_e.as<std::uint32_t>();
-  BFN_HIP(fill_launch(a.arena_edges, total, kNone, s));
-  BFN_HIP(paths_launch(a, ws->Q, s));
-  if (total) {
-    BFN_HIP(hipMemcpyAsync(vertices, ws->arena_v.ptr, 4ull * total, hipMemcpyDeviceToHost, s));
-    BFN_HIP(hipMemcpyAsync(labels, ws->arena_l.ptr, 4ull * total, hipMemcpyDeviceToHost, s));
-    BFN_HIP(hipMemcpyAsync(edge_ids, ws->arena_e.ptr, 4ull * total, hipMemcpyDeviceToHost, s));
+  if (!ws->paths_emitted) {
+    BFN_HIP(make_room(total + total / 4));
+    BFN_HIP(emit());
+    BFN_HIP(hipStreamSynchronize(s));
+    ws->paths_emitted = true;
   }
-  BFN_HIP(hipStreamSynchronize(s));
+  const std::uint32_t* ha = ws->h_arena.as<std::uint32_t>();
+  std::memcpy(vertices, ha, 4ull * total);
+  std::memcpy(labels, ha + ws->arena_room, 4ull * total);
+  std::memcpy(edge_ids, ha + 2 * ws->arena_room, 4ull * total);
   ws->have_paths = true;
   ws->arena_vertices = total;
   return BFN_OK;

@@ -340,7 +340,7 @@ int32_t bfn_batch_run_static(bfn_graph graph, const bfn_batch_desc* d, const bfn
       if (done) break;
     }
   }
-  BFN_HIP_STATIC(finalize_launch(gv, b, nullptr, m + o_status, s));
+  BFN_HIP_STATIC(finalize_launch(gv, b, nullptr, m + o_status, nullptr, s));
   hipLaunchKernelGGL(static_targets_kernel, dim3((Q + 127) / 128), dim3(128), 0, s, gv, b, u32(o_targets));
   BFN_HIP_STATIC(hipGetLastError());
   static_assert(sizeof(bfn_query_status) == sizeof(QueryStatusDev), "per-query status layout");

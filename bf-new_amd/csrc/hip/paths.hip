@@ -5,13 +5,25 @@
 // compact_path_results.hip.cpp:169-249): from each target, walk tight
 // admitted incoming edges (d[u] + w == d[v], u selected and finite) in
 // stable-EdgeId order, skipping vertices already on the path, backtracking
-// when a vertex has no untried candidate, until a source is reached.  Here
-// one wavefront owns one query: its 64 lanes scan a vertex's incoming edges
-// together and a wave min-reduction picks the smallest untried EdgeId, so a
-// step costs one pass over the in-edges instead of a sort.  A frame stores
-// its vertex and the last EdgeId tried from it; resuming a frame asks for the
-// smallest candidate above that EdgeId, which visits candidates in exactly
-// the reference's cursor order.
+// when a vertex has no untried candidate, until a source is reached.  A
+// workgroup owns a query and a wave one target: its 64 lanes scan a vertex's
+// incoming edges together and a wave min-reduction picks the smallest
+// EdgeId, so a step costs one pass over the in-edges instead of a sort.
+//
+// Where every tight edge lowers the label (no zero-weight plateau), the walk
+// never meets its own path and never runs dry, so it is a chain of smallest
+// EdgeIds: walk_descending.  It is bound by the latency of a step's dependent
+// reads, so the winning lane hands over all that the next step needs (slot,
+// label, column bounds) and a step is four dependent reads; looking the
+// vertex up in its query's tiles three times per step made it about thirty.
+// The first pass keeps each path in the frame scratch, so the second only
+// copies it out.  A whole routing pass, before and after: one net on 64x64x256
+// tiles 491 -> 384 us, 41 queries with 123 targets on 45x37x301 1168 -> 905
+// us, 256 queries on 128x128x512 14.35 -> 13.97 ms.  A target whose walk meets a plateau, a dead end or the end
+// of its frame space is walked again by walk_backtracking, the general rule:
+// a frame stores its vertex and the last EdgeId tried from it; resuming a
+// frame asks for the smallest candidate above that EdgeId, which visits
+// candidates in exactly the reference's cursor order.
 #include "bfn_internal.hpp"
 
 namespace bfn {
@@ -43,6 +55,14 @@ __device__ __forceinline__ bool is_source(const DevBatch& b, std::uint32_t q, st
   return find_sorted(b.sources, b.source_offsets[q], b.source_offsets[q + 1], v) != kNone;
 }
 
+// The lanes of this wave meet, and their global stores are visible to its own
+// later loads (in uniform control flow).
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_s_waitcnt(0);
+  __threadfence_block();
+  (void)__ballot(1);
+}
+
 __device__ __forceinline__ unsigned long long wave_min_u64(unsigned long long x) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -54,132 +74,261 @@ __device__ __forceinline__ unsigned long long wave_min_u64(unsigned long long x)
   return x;
 }
 
-// One 64-lane block per query.
-__global__ __launch_bounds__(64) void compact_paths_kernel(PathArgs a) {
+// Pool offset of slot s's final labels.
+__device__ __forceinline__ unsigned long long labels_of_slot(const DevGraph& g, const DevBatch& b,
+                                                             std::uint32_t s, std::uint32_t col) {
+  if (b.slot_desc) {
+    const unsigned long long at = (static_cast<unsigned long long>(b.slot_desc[s].dist_hi) << 32) |
+                                  b.slot_desc[s].dist_lo;
+    return at + static_cast<unsigned long long>(col) * b.slot_desc[s].npt;
+  }
+  unsigned long long at = b.slot_dist[s];
+  if (col) {
+    const std::uint32_t T = b.tiles[s];
+    at += g.tile_vertex_offsets[T + 1] - g.tile_vertex_offsets[T];
+  }
+  return at;
+}
+
+// Frames [fb, fb + room) hold the walk: vertex, the edge it was reached by,
+// and its label.  Returns the number of edges, or -1 when the target needs
+// walk_backtracking.  Wave-uniform arguments and result.
+__device__ std::int32_t walk_descending(const PathArgs& a, std::uint32_t q, std::uint32_t target,
+                                        std::uint32_t col, unsigned long long fb,
+                                        unsigned long long room) {
+  const DevGraph& g = a.g;
+  const DevBatch& b = a.b;
+  const std::uint32_t lane = threadIdx.x & 63u;
+  const std::uint32_t T = g.owner_tiles[target];
+  const std::uint32_t s = find_slot(b, q, T);
+  std::uint32_t v = target;
+  std::uint32_t dv = b.dist[labels_of_slot(g, b, s, col) + (target - g.tile_vertex_offsets[T])];
+  std::uint32_t c0 = g.column_offsets[v], c1 = g.column_offsets[v + 1], in_base = b.slot_in_base[s];
+  if (lane == 0) {
+    a.frame_vertex[fb] = v;
+    a.frame_via[fb] = kNone;
+    a.frame_last[fb] = dv;
+  }
+  for (std::int32_t top = 0;; ++top) {
+    if (dv == 0u && is_source(b, q, v)) return top;
+    if (static_cast<unsigned long long>(top) + 1 >= room) return -1;
+    std::uint32_t eid = kNone, u = 0, du = 0, u0 = 0, u1 = 0, u_base = 0;
+    bool plateau = false;
+    for (std::uint32_t e = c0 + lane; e < c1; e += 64) {
+      const std::uint32_t id = g.in_edge_ids[e];
+      const std::uint32_t p = g.csc_pack[e];
+      const std::uint32_t from = g.sources[e];
+      const float w = g.in_weights[e];
+      const std::uint32_t ns = b.slot_in[in_base + (p >> 24)];
+      if (ns == kNone) continue;
+      // what the next step needs of this candidate travels with its label
+      const std::uint32_t n0 = g.column_offsets[from], n1 = g.column_offsets[from + 1];
+      const std::uint32_t n_base = b.slot_in_base[ns];
+      const std::uint32_t d = b.dist[labels_of_slot(g, b, ns, col) + ((p >> 12) & kPackLocalMask)];
+      if (d == kInfBits || as_bits(as_float(d) + w) != dv) continue;
+      plateau |= d == dv;
+      if (id < eid) {
+        eid = id;
+        u = from;
+        du = d;
+        u0 = n0;
+        u1 = n1;
+        u_base = n_base;
+      }
+    }
+    std::uint32_t best = eid;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) best = min(best, __shfl_xor(best, off));
+    if (best == kNone || __ballot(plateau)) return -1;
+    const unsigned long long m = __ballot(eid == best);
+    const int winner = __popcll((m - 1ull) & ~m);  // an edge has one id: one lane holds it
+    v = __shfl(u, winner);
+    dv = __shfl(du, winner);
+    c0 = __shfl(u0, winner);
+    c1 = __shfl(u1, winner);
+    in_base = __shfl(u_base, winner);
+    if (lane == 0) {
+      a.frame_vertex[fb + top + 1] = v;
+      a.frame_via[fb + top + 1] = best;
+      a.frame_last[fb + top + 1] = dv;
+    }
+  }
+}
+
+// The general walk of one target by one wave, in the query's whole frame
+// space and with its own stamp on the vertices of its path.  Returns the
+// number of edges, or -1 when no tight path reaches a source.
+__device__ std::int32_t walk_backtracking(const PathArgs& a, std::uint32_t q, std::uint32_t target,
+                                          std::uint32_t stamp, std::uint32_t copy,
+                                          unsigned long long fb) {
+  const DevGraph& g = a.g;
+  const DevBatch& b = a.b;
+  const std::uint32_t lane = threadIdx.x & 63u;
+  unsigned long long target_pool;
+  label_of(g, b, q, target, copy, &target_pool);
+  std::int32_t top = 0;
+  std::uint32_t v = target;
+  std::uint32_t last = kNone;  // EdgeId last tried from the top frame
+  if (lane == 0) {
+    a.frame_vertex[fb] = target;
+    a.frame_via[fb] = kNone;
+    a.onpath[target_pool] = stamp;
+  }
+  for (;;) {
+    if (is_source(b, q, v)) return top;
+    const std::uint32_t T = g.owner_tiles[v];
+    const std::uint32_t s = find_slot(b, q, T);
+    const std::uint32_t dv = label_of(g, b, q, v, copy, nullptr);
+    const std::uint32_t in0 = g.in_nbr_offsets[T];
+    unsigned long long best = ~0ull;
+    for (std::uint32_t e = g.column_offsets[v] + lane; e < g.column_offsets[v + 1]; e += 64) {
+      const std::uint32_t eid = g.in_edge_ids[e];
+      if (last != kNone && eid <= last) continue;
+      const std::uint32_t p = g.csc_pack[e];
+      const std::uint32_t k = p >> 24;
+      const std::uint32_t ns = b.slot_in[b.slot_in_base[s] + k];
+      if (ns == kNone) continue;
+      const std::uint32_t nt = g.in_nbr_tiles[in0 + k];
+      const std::uint32_t nn = g.tile_vertex_offsets[nt + 1] - g.tile_vertex_offsets[nt];
+      const unsigned long long pool = b.slot_dist[ns] + ((p >> 12) & kPackLocalMask);
+      const std::uint32_t du =
+          b.dist[pool + static_cast<unsigned long long>(column_of(b, q, copy)) * nn];
+      if (du == kInfBits) continue;
+      if (as_bits(as_float(du) + g.in_weights[e]) != dv) continue;
+      if (a.onpath[pool] == stamp) continue;
+      const unsigned long long key =
+          (static_cast<unsigned long long>(eid) << 32) | g.sources[e];
+      best = key < best ? key : best;
+    }
+    best = wave_min_u64(best);
+    if (best != ~0ull) {
+      const std::uint32_t eid = static_cast<std::uint32_t>(best >> 32);
+      const std::uint32_t u = static_cast<std::uint32_t>(best);
+      unsigned long long upool;
+      label_of(g, b, q, u, copy, &upool);
+      if (lane == 0) {
+        a.frame_last[fb + top] = eid;
+        a.frame_vertex[fb + top + 1] = u;
+        a.frame_via[fb + top + 1] = eid;
+        a.onpath[upool] = stamp;
+      }
+      ++top;
+      v = u;
+      last = kNone;
+    } else {
+      unsigned long long vpool;
+      label_of(g, b, q, v, copy, &vpool);
+      if (lane == 0) a.onpath[vpool] = 0;
+      --top;
+      if (top < 0) return -1;
+      wave_fence();
+      v = a.frame_vertex[fb + top];
+      last = a.frame_last[fb + top];
+    }
+    wave_fence();
+  }
+}
+
+// One workgroup per query, wave w walks (pass 1) or copies out (pass 2) its
+// targets w, w + waves, ...; wave 0 then takes those that need backtracking.
+__global__ __launch_bounds__(512) void compact_paths_kernel(PathArgs a) {
   const std::uint32_t q = a.query_list ? a.query_list[blockIdx.x] : blockIdx.x;
   const DevGraph& g = a.g;
   const DevBatch& b = a.b;
-  const std::uint32_t lane = threadIdx.x;
+  const std::uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
   const std::uint32_t copy =
       a.jacobi_copy_from_control ? (b.control->round & 1u) : a.jacobi_copy;
+  const std::uint32_t col = column_of(b, q, copy);
+  const std::uint32_t t0 = b.target_offsets[q], t1 = b.target_offsets[q + 1];
   const unsigned long long fb = a.frame_base[q];
-  for (std::uint32_t t = b.target_offsets[q]; t < b.target_offsets[q + 1]; ++t) {
-    const std::uint32_t target = b.targets[t];
-    unsigned long long target_pool;
-    const std::uint32_t dt = label_of(g, b, q, target, copy, &target_pool);
+  const unsigned long long space =
+      a.frame_slab ? static_cast<unsigned long long>(b.tile_end[q] - b.tile_begin[q]) * a.frame_slab
+                   : (q + 1 < b.query_count ? a.frame_base[q + 1] : a.frame_words) - fb;
+  const unsigned long long room = space / (t1 - t0);  // frames of one target's descending walk
+  const std::uint32_t state = a.query_clean[q];
+  auto summarise = [&](std::uint32_t t, std::uint32_t target, std::uint32_t dt, std::int32_t top,
+                       unsigned long long frames) {
+    if (lane != 0) return;
     std::uint32_t* sum = a.summaries + static_cast<std::size_t>(t) * 7;
-    if (!a.query_clean[q] || dt == kInfBits) {
-      if (a.pass == 1 && lane == 0) {
-        sum[0] = target;
-        sum[1] = 0;
-        sum[2] = kInfBits;
-        sum[3] = 0;
-        sum[4] = 0;                                  // not_reached
-        sum[5] = a.query_clean[q] ? 1u : 2u;         // unreachable / terminal failure
-        sum[6] = 0;
-        a.lengths[t] = 0;
+    const bool reached = dt != kInfBits && (state & kPathClean);
+    const bool found = reached && top >= 0;
+    sum[0] = target;
+    sum[1] = found ? a.frame_vertex[frames + top] : 0u;
+    sum[2] = reached ? dt : kInfBits;
+    sum[3] = found ? static_cast<std::uint32_t>(top) : 0u;
+    sum[4] = reached;
+    // complete, query terminal failure, unreachable, no tight path
+    sum[5] = found ? 0u : !(state & kPathClean) ? 2u : dt == kInfBits ? 1u : 3u;
+    sum[6] = found;
+    a.lengths[t] = found ? static_cast<unsigned long long>(top) + 1 : 0ull;
+  };
+  // Edges share the vertex offsets; a path of L edges leaves slot L unused.
+  auto copy_out = [&](std::uint32_t t, std::int32_t top, unsigned long long frames, bool labels) {
+    const unsigned long long out = a.offsets[t];
+    for (std::int32_t i = static_cast<std::int32_t>(lane); i <= top; i += 64) {
+      const unsigned long long from = frames + static_cast<std::uint32_t>(top - i);
+      const std::uint32_t vert = a.frame_vertex[from];
+      const std::uint32_t label = labels ? a.frame_last[from] : label_of(g, b, q, vert, copy, nullptr);
+      const std::uint32_t edge = i < top ? a.frame_via[from] : kNone;
+      a.arena_vertices[out + i] = vert;
+      a.arena_labels[out + i] = label;
+      a.arena_edges[out + i] = edge;
+      if (a.host_vertices) {
+        a.host_vertices[out + i] = vert;
+        a.host_labels[out + i] = label;
+        a.host_edges[out + i] = edge;
       }
-      continue;
     }
-    const std::uint32_t stamp = a.stamp_base + t + 1;
-    std::int32_t top = 0;
-    std::uint32_t v = target;
-    std::uint32_t last = kNone;  // EdgeId last tried from the top frame
-    if (lane == 0) {
-      a.frame_vertex[fb] = target;
-      a.frame_via[fb] = kNone;
-      a.onpath[target_pool] = stamp;
-    }
-    bool found_source = false;
-    for (;;) {
-      if (is_source(b, q, v)) {
-        found_source = true;
-        break;
+  };
+  const bool emit = a.pass == 2;
+  if (emit && a.arena_capacity != ~0ull && a.offsets[a.target_total] > a.arena_capacity)
+    return;  // the host retries with room for them
+  __shared__ std::uint32_t general;  // targets for walk_backtracking
+  if (threadIdx.x == 0) general = 0;
+  __syncthreads();
+  if (!emit || !(state & kPathGeneral)) {
+    for (std::uint32_t t = t0 + wave; t < t1; t += waves) {
+      const std::uint32_t target = b.targets[t];
+      const unsigned long long frames = fb + room * (t - t0);
+      if (emit) {
+        const std::int32_t n = static_cast<std::int32_t>(a.lengths[t]);
+        if (n) copy_out(t, n - 1, frames, true);
+        continue;
       }
-      const std::uint32_t T = g.owner_tiles[v];
-      const std::uint32_t s = find_slot(b, q, T);
-      const std::uint32_t dv = label_of(g, b, q, v, copy, nullptr);
-      const std::uint32_t in0 = g.in_nbr_offsets[T];
-      unsigned long long best = ~0ull;
-      for (std::uint32_t e = g.column_offsets[v] + lane; e < g.column_offsets[v + 1]; e += 64) {
-        const std::uint32_t eid = g.in_edge_ids[e];
-        if (last != kNone && eid <= last) continue;
-        const std::uint32_t p = g.csc_pack[e];
-        const std::uint32_t k = p >> 24;
-        const std::uint32_t ns = b.slot_in[b.slot_in_base[s] + k];
-        if (ns == kNone) continue;
-        const std::uint32_t nt = g.in_nbr_tiles[in0 + k];
-        const std::uint32_t nn = g.tile_vertex_offsets[nt + 1] - g.tile_vertex_offsets[nt];
-        const unsigned long long pool = b.slot_dist[ns] + ((p >> 12) & kPackLocalMask);
-        const std::uint32_t du =
-            b.dist[pool + static_cast<unsigned long long>(column_of(b, q, copy)) * nn];
-        if (du == kInfBits) continue;
-        if (as_bits(as_float(du) + g.in_weights[e]) != dv) continue;
-        if (a.onpath[pool] == stamp) continue;
-        const unsigned long long key =
-            (static_cast<unsigned long long>(eid) << 32) | g.sources[e];
-        best = key < best ? key : best;
-      }
-      best = wave_min_u64(best);
-      __syncthreads();
-      if (best != ~0ull) {
-        const std::uint32_t eid = static_cast<std::uint32_t>(best >> 32);
-        const std::uint32_t u = static_cast<std::uint32_t>(best);
-        unsigned long long upool;
-        label_of(g, b, q, u, copy, &upool);
-        if (lane == 0) {
-          a.frame_last[fb + top] = eid;
-          a.frame_vertex[fb + top + 1] = u;
-          a.frame_via[fb + top + 1] = eid;
-          a.onpath[upool] = stamp;
-        }
-        ++top;
-        v = u;
-        last = kNone;
-      } else {
-        unsigned long long vpool;
-        label_of(g, b, q, v, copy, &vpool);
-        if (lane == 0) a.onpath[vpool] = 0;
-        --top;
-        if (top < 0) break;
-        __threadfence_block();
-        __syncthreads();
-        v = a.frame_vertex[fb + top];
-        last = a.frame_last[fb + top];
-      }
-      __threadfence_block();
-      __syncthreads();
-    }
-    if (a.pass == 1) {
-      if (lane == 0) {
-        sum[0] = target;
-        sum[2] = dt;
-        sum[4] = 1;  // reached
-        if (found_source) {
-          sum[1] = a.frame_vertex[fb + top];
-          sum[3] = static_cast<std::uint32_t>(top);
-          sum[5] = 0;  // complete
-          sum[6] = 1;
-          a.lengths[t] = static_cast<unsigned long long>(top) + 1;
-        } else {
-          sum[1] = 0;
-          sum[3] = 0;
-          sum[5] = 3;  // no_tight_path
-          sum[6] = 0;
-          a.lengths[t] = 0;
+      const std::uint32_t dt = label_of(g, b, q, target, copy, nullptr);
+      std::int32_t top = -1;
+      if (dt != kInfBits && (state & kPathClean)) {
+        top = room ? walk_descending(a, q, target, col, frames, room) : -1;
+        if (top < 0) {
+          if (lane == 0) {
+            atomicAdd(&general, 1u);
+            a.lengths[t] = ~0ull;
+          }
+          continue;
         }
       }
-    } else if (found_source) {
-      // Edges share the vertex offsets; a path of L edges leaves slot L unused.
-      const unsigned long long out = a.offsets[t];
-      for (std::int32_t i = lane; i <= top; i += 64) {
-        const std::uint32_t vert = a.frame_vertex[fb + (top - i)];
-        a.arena_vertices[out + i] = vert;
-        a.arena_labels[out + i] = label_of(g, b, q, vert, copy, nullptr);
-        if (i < top) a.arena_edges[out + i] = a.frame_via[fb + (top - i)];
-      }
+      wave_fence();
+      summarise(t, target, dt, top, frames);
     }
+    wave_fence();
     __syncthreads();
+    if (emit) return;
+    const std::uint32_t marked = general ? state | kPathGeneral : state & ~kPathGeneral;
+    if (threadIdx.x == 0 && marked != state) a.query_clean[q] = marked;
+    if (general == 0) return;
+  }
+  if (wave != 0) return;
+  for (std::uint32_t t = t0; t < t1; ++t) {
+    const std::uint32_t target = b.targets[t];
+    if (a.lengths[t] != (emit ? a.lengths[t] : ~0ull) || a.lengths[t] == 0) continue;
+    const std::int32_t top = walk_backtracking(a, q, target, a.stamp_base + t + 1, copy, fb);
+    wave_fence();
+    if (emit) {
+      if (top >= 0) copy_out(t, top, fb, false);
+    } else {
+      summarise(t, target, label_of(g, b, q, target, copy, nullptr), top, fb);
+    }
+    wave_fence();
   }
 }
 
@@ -236,7 +385,7 @@ __global__ void scatter_distances_kernel(DevGraph g, DevBatch b, std::uint32_t q
 
 
 __global__ void finalize_kernel(DevGraph g, DevBatch b, const unsigned long long* relaxations,
-                                QueryStatusDev* out) {
+                                QueryStatusDev* out, std::uint32_t* path_state) {
   const std::uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
   if (q >= b.query_count) return;
   const DevControl* c = b.control;
@@ -260,6 +409,7 @@ __global__ void finalize_kernel(DevGraph g, DevBatch b, const unsigned long long
   st.error_bits = c->error_bits;
   st.engine = b.engine[q];
   out[q] = st;
+  if (path_state) path_state[q] = converged ? kPathClean : 0u;  // what the path passes start from
 }
 
 // Work-normalised relaxation count: admitted out-edges of reached vertices.
@@ -334,8 +484,11 @@ __global__ void scan_u64_kernel(const unsigned long long* in, unsigned long long
 }
 
 // ---- launch wrappers ------------------------------------------------------
+// A wave per target up to eight (the walks of a query's targets are chains of
+// their own; more waves per workgroup than targets would only exit).
 hipError_t paths_launch(const PathArgs& a, std::uint32_t query_count, hipStream_t stream) {
-  hipLaunchKernelGGL(compact_paths_kernel, dim3(query_count), dim3(64), 0, stream, a);
+  const std::uint32_t waves = a.most_targets < 1 ? 1u : a.most_targets > 8 ? 8u : a.most_targets;
+  hipLaunchKernelGGL(compact_paths_kernel, dim3(query_count), dim3(64 * waves), 0, stream, a);
   return hipGetLastError();
 }
 
@@ -390,9 +543,10 @@ hipError_t gather_region_launch(const DevGraph& g, const DevBatch& b, std::uint3
 }
 
 hipError_t finalize_launch(const DevGraph& g, const DevBatch& b,
-                           const unsigned long long* relaxations, void* out, hipStream_t stream) {
+                           const unsigned long long* relaxations, void* out,
+                           std::uint32_t* path_state, hipStream_t stream) {
   hipLaunchKernelGGL(finalize_kernel, dim3((b.query_count + 127) / 128), dim3(128), 0, stream, g,
-                     b, relaxations, static_cast<QueryStatusDev*>(out));
+                     b, relaxations, static_cast<QueryStatusDev*>(out), path_state);
   return hipGetLastError();
 }
 

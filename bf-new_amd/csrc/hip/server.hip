@@ -366,6 +366,9 @@ hipError_t bfn_server_s::step(std::uint32_t admit_count, std::uint32_t tile_coun
     a.query_clean = d_clean;
     a.query_list = d_done + 1;
     a.frame_base = d_frame_base;
+    a.frame_words = static_cast<std::uint64_t>(Scap) * max_v;
+    a.frame_slab = max_v;
+    a.most_targets = 1;
     a.frame_vertex = d_frames;
     a.frame_last = d_frames + static_cast<std::size_t>(Scap) * max_v;
     a.frame_via = a.frame_last + static_cast<std::size_t>(Scap) * max_v;
@@ -395,6 +398,7 @@ hipError_t bfn_server_s::step(std::uint32_t admit_count, std::uint32_t tile_coun
       a.pass = 2;
       a.stamp_base = Qcap;
       a.offsets = d_path_offsets;
+      a.arena_capacity = ~0ull;  // sized from the offsets above
       a.arena_vertices = d_arena_v;
       a.arena_labels = d_arena_l;
       a.arena_edges = d_arena_e;
