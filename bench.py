@@ -492,8 +492,11 @@ def main():
                                           boundary_mode=tune["boundary_mode"],
                                           min_waves=tune["min_waves"], **scheduling(tune)))
     elapsed, relax_ms, launches, paths_ms = timed_steps(ws, args.steps, args.warmup, paths=True)
-    # one round kernel + one advance kernel per host-polled or replayed round
-    round_launches = 1 if tune["control"] == bfn.PERSISTENT and not tune["use_graph"] else launches // 2
+    # one round kernel per host-polled or replayed round, and with slot-order
+    # claims one compaction kernel
+    per_round = 2 if tune["claim_order"] else 1
+    round_launches = (1 if tune["control"] == bfn.PERSISTENT and not tune["use_graph"]
+                      else launches // per_round)
     value = relax_per_step * args.steps / elapsed
     ms_per_step = elapsed * 1e3 / args.steps
     kernel_ms = float(np.mean(relax_ms))

@@ -429,6 +429,23 @@ __device__ __forceinline__ bool grid_barrier_flat(DevControl* c, std::uint32_t b
   return __syncthreads_or(!ok) == 0;
 }
 
+// Arrival of a workgroup (one thread of it) on its group's counter, and of
+// the group's last on the top one; whether it was the last of the grid.
+// Every counter is back at zero by then.
+template <std::uint32_t G = kArrivalGroups>
+__device__ __forceinline__ bool arrive_last(DevControl* c, std::uint32_t blocks) {
+  const std::uint32_t g = blockIdx.x % G;
+  const std::uint32_t members = (blocks + G - 1u - g) / G;
+  const std::uint32_t groups = blocks < G ? blocks : G;
+  std::uint32_t* mine = &c->group_arrivals[g * kBarrierStride];
+  if (atomic_add_agent(mine, 1u) != members - 1) return false;
+  store_agent(mine, 0u);
+  __builtin_amdgcn_s_waitcnt(0);
+  if (atomic_add_agent(&c->barrier_count, 1u) != groups - 1) return false;
+  store_agent(&c->barrier_count, 0u);
+  return true;
+}
+
 // Two-level: a workgroup arrives on its group's counter (group =
 // blockIdx % G; G is a multiple of 8, so every group's workgroups sit on the
 // XCD that the dispatcher's round-robin placed them on); the last arriver of
@@ -449,18 +466,7 @@ __device__ __forceinline__ bool grid_barrier_grouped(DevControl* c, std::uint32_
   if (threadIdx.x == 0) {
     const std::uint32_t gen = load_agent(&c->barrier_generation);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    const std::uint32_t g = blockIdx.x % G;
-    const std::uint32_t members = (blocks + G - 1u - g) / G;
-    const std::uint32_t groups = blocks < G ? blocks : G;
-    std::uint32_t* mine = &c->group_arrivals[g * kBarrierStride];
-    bool last = false;
-    if (atomic_add_agent(mine, 1u) == members - 1) {
-      store_agent(mine, 0u);
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-      last = atomic_add_agent(&c->barrier_count, 1u) == groups - 1;
-    }
-    if (last) {
-      store_agent(&c->barrier_count, 0u);
+    if (arrive_last<G>(c, blocks)) {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
       store_agent(&c->barrier_generation, gen + 1);
     } else {

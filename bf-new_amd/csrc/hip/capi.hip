@@ -4,10 +4,10 @@
 //   persistent_cooperative -- one hipLaunchCooperativeKernel runs every round
 //                             with a grid barrier between rounds
 //                             (batched_jacobi.hip.cpp:838-878 shape);
-//   chunked / per_round    -- rounds_per_chunk (round kernel + one-thread
-//                             advance) pairs, then one controller copy and
-//                             stream sync (batched_jacobi.hip.cpp:1540-1587);
-//   bfn_tuning.use_graph   -- graph_rounds round pairs and the controller
+//   chunked / per_round    -- rounds_per_chunk round kernels, then one
+//                             controller copy and stream sync
+//                             (batched_jacobi.hip.cpp:1540-1587);
+//   bfn_tuning.use_graph   -- graph_rounds round kernels and the controller
 //                             copy captured once into a hipGraph and replayed
 //                             after the preparation launches; rounds beyond
 //                             convergence exit at their first instruction,
@@ -884,6 +884,7 @@ int32_t run_resident_batch(bfn_workspace ws) {
   ws->paths_counted = ws->paths_emitted = false;
   BFN_HIP(hipEventRecord(ws->ev_start, s));
   const bool graph_mode = t.use_graph && o.control_mode != 0;
+  const std::uint64_t per_round = b.ordered ? 2u : 1u;  // the round and, in slot order, the compaction
   unsigned long long* relax = t.count_relaxations ? ws->relax.as<unsigned long long>() : nullptr;
   auto finalize = [&]() -> hipError_t {
     hipError_t e = hipSuccess;
@@ -941,7 +942,7 @@ int32_t run_resident_batch(bfn_workspace ws) {
     ws->slots_resolved = true;
     BFN_HIP(hipEventRecord(ws->ev_relax0, s));
     BFN_HIP(hipGraphLaunch(ws->graph_exec, s));
-    ws->launches += 2ull * rounds;
+    ws->launches += per_round * rounds;
     BFN_HIP(hipStreamSynchronize(s));
     ++ws->host_syncs;
     ++ws->controller_copies;
@@ -953,7 +954,7 @@ int32_t run_resident_batch(bfn_workspace ws) {
       for (std::uint32_t r = 0; r < chunk; ++r)
         BFN_HIP(relax_launch(ws->block, false, false, ws->grid, ws->lds_bytes, ws->max_v,
                              ws->work_words, g->view, b, s));
-      ws->launches += 2ull * chunk;
+      ws->launches += per_round * chunk;
       BFN_HIP(hipMemcpyAsync(ws->h_control.ptr, ws->control.ptr, kControlHead,
                              hipMemcpyDeviceToHost, s));
       BFN_HIP(hipStreamSynchronize(s));
@@ -980,7 +981,7 @@ int32_t run_resident_batch(bfn_workspace ws) {
       for (std::uint32_t r = 0; r < chunk; ++r)
         BFN_HIP(relax_launch(ws->block, false, false, ws->grid, ws->lds_bytes, ws->max_v,
                              ws->work_words, g->view, b, s));
-      ws->launches += 2ull * chunk;
+      ws->launches += per_round * chunk;
       BFN_HIP(hipMemcpyAsync(ws->h_control.ptr, ws->control.ptr, kControlHead,
                              hipMemcpyDeviceToHost, s));
       BFN_HIP(hipStreamSynchronize(s));

@@ -1,48 +1,17 @@
-// relax.hip -- control of the relaxation engines: the advance kernels
-// between round launches, batch preparation (control reset, label fill,
+// relax.hip -- control of the relaxation engines: the compaction between
+// slot-order rounds, batch preparation (control reset, label fill,
 // slot tables, seeds) and the launch dispatch to the kernel variant of a
 // batch's engine set (relax_kernels.hpp, instantiated by relax_mixed.hip,
 // relax_push.hip, relax_push_lds.hip and relax_pull.hip).
 #include "bfn_launch.hpp"
 
+#include <algorithm>
 #include <mutex>
 
 namespace bfn {
 
-// One wave: lane x looks after class x of the lists.
-__global__ __launch_bounds__(64) void relax_advance_kernel(DevBatch b) {
-  static_assert(kQueueClasses == 64, "one lane per class");
-  DevControl* c = b.control;
-  if (c->done) return;
-  const std::uint32_t lane = threadIdx.x;
-  const std::uint32_t r = c->round;
-  const bool queued = *list_count(b, (r + 1) % 3, lane) != 0;
-  const bool any = __ballot(queued) != 0;
-  if (b.instrumentation) {
-    std::uint32_t n = *list_count(b, r % 3, lane);
-    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off);
-    if (lane == 0 && n > c->max_list) c->max_list = n;
-  }
-  *list_count(b, (r + 2) % 3, lane) = 0;
-  *list_claim(b, (r + 2) % 3, lane) = 0;
-  if (lane != 0) return;
-  if (b.prio) {
-    c->window_limit = next_window_limit(c, b, r, c->window_limit);
-    reset_next_min(c, (r + 2) % 3);
-  }
-  c->round = r + 1;
-  c->rounds_executed = r + 1;
-  if (!any) {
-    c->done = 1;
-    c->stop_reason = kStopConverged;
-  } else if (b.maximum_rounds && r + 1 >= b.maximum_rounds) {
-    c->done = 1;
-    c->stop_reason = kStopMaximumRounds;
-  }
-}
-
 // Between rounds in slot order (one workgroup): count the round as
-// relax_advance_kernel does, then compact the queued bits into lists[0, n)
+// advance_round does, then compact the queued bits into lists[0, n)
 // and clear them.  Slots are taken in groups of 64 (two bit words); group k
 // belongs to segment k % 8, and the list holds segment 0's groups in order,
 // then segment 1's, ..., so each segment is in slot order.  first = 1 (after
@@ -144,9 +113,8 @@ __global__ __launch_bounds__(1024) void ordered_advance_kernel(DevBatch b, std::
 // ---------------------------------------------------------------------------
 // Batch preparation.
 // ---------------------------------------------------------------------------
-// One workgroup.
-__global__ __launch_bounds__(1024) void reset_control_kernel(DevControl* c, std::uint32_t* queue,
-                                                             std::uint32_t window) {
+// Control block and list counters of a run, by one workgroup.
+__device__ __forceinline__ void reset_control(DevControl* c, std::uint32_t* queue, std::uint32_t window) {
   std::uint32_t* words = reinterpret_cast<std::uint32_t*>(c);
   for (std::uint32_t i = threadIdx.x; i < sizeof(DevControl) / 4; i += blockDim.x) words[i] = 0;
   if (queue)
@@ -158,6 +126,11 @@ __global__ __launch_bounds__(1024) void reset_control_kernel(DevControl* c, std:
   if (threadIdx.x == 0) c->window_limit = window;  // round 0 visits the sources' slots (priority 0)
 }
 
+__global__ __launch_bounds__(1024) void reset_control_kernel(DevControl* c, std::uint32_t* queue,
+                                                             std::uint32_t window) {
+  reset_control(c, queue, window);
+}
+
 __global__ void fill_u32_kernel(std::uint32_t* p, unsigned long long n, std::uint32_t v) {
   const unsigned long long stride = static_cast<unsigned long long>(gridDim.x) * blockDim.x;
   for (unsigned long long i = static_cast<unsigned long long>(blockIdx.x) * blockDim.x +
@@ -166,64 +139,89 @@ __global__ void fill_u32_kernel(std::uint32_t* p, unsigned long long n, std::uin
     p[i] = v;
 }
 
-// Per run: each slot's queue stamp, window priority and its query's last
-// change, and the engine-set check.  With `structure` (the first run of a
-// batch) also the slot's in/out neighbour tiles resolved to the query's
-// slots and its descriptor: they depend only on the batch and the graph's
-// tile directory, so the reruns of a batch keep them.
-__global__ void prep_slots_kernel(DevGraph g, DevBatch b, std::uint32_t structure) {
-  const std::uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+// Preparation of a run, one launch: the first `fill_blocks` workgroups set
+// every label to +inf, the next `slot_blocks` the slots' queue stamps and
+// window priorities, the last one the control block and each query's last
+// change.  With `structure` (the first run of a batch) the slot workgroups
+// also resolve each slot's in- and out-neighbour tiles to the query's slots
+// and write its descriptor: they depend only on the batch and the graph's
+// tile directory, so the reruns of a batch keep them.  A neighbour is a
+// binary search of dependent reads, so kSlotLanes lanes share a slot's
+// lists; one thread per slot took 27 us for 36 slots and 181 us for 213k.
+constexpr std::uint32_t kSlotLanes = 16;
+
+__global__ __launch_bounds__(256) void prepare_kernel(DevGraph g, DevBatch b, unsigned long long pool_words,
+                                                      std::uint32_t fill_blocks, std::uint32_t slot_blocks,
+                                                      std::uint32_t structure) {
+  const std::uint32_t tid = threadIdx.x;
+  if (blockIdx.x < fill_blocks) {
+    const uint4 inf = make_uint4(kInfBits, kInfBits, kInfBits, kInfBits);
+    const unsigned long long quads = pool_words / 4;
+    const unsigned long long stride = static_cast<unsigned long long>(fill_blocks) * 256;
+    for (unsigned long long i = static_cast<unsigned long long>(blockIdx.x) * 256 + tid; i < quads; i += stride)
+      reinterpret_cast<uint4*>(b.dist)[i] = inf;
+    if (blockIdx.x == 0 && tid < pool_words % 4) b.dist[4 * quads + tid] = kInfBits;
+    return;
+  }
+  if (blockIdx.x >= fill_blocks + slot_blocks) {
+    reset_control(b.control, b.queue, b.window);
+    for (std::uint32_t q = tid; q < b.query_count; q += 256) b.last_change[q] = 0;
+    return;
+  }
+  const std::uint32_t lanes = structure ? kSlotLanes : 1u;
+  const std::uint32_t s = (blockIdx.x - fill_blocks) * (256u / lanes) + tid / lanes;
+  const std::uint32_t lane = tid % lanes;
   if (s >= b.slot_count) return;
-  const std::uint32_t q = b.slot_query[s];
-  if (structure) {
-    const std::uint32_t T = b.tiles[s];
-    const std::uint32_t in0 = g.in_nbr_offsets[T], in1 = g.in_nbr_offsets[T + 1];
-    const std::uint32_t ib = b.slot_in_base[s];
-    for (std::uint32_t k = in0; k < in1; ++k)
-      b.slot_in[ib + (k - in0)] = find_slot(b, q, g.in_nbr_tiles[k]);
-    const std::uint32_t o0 = g.out_nbr_offsets[T], o1 = g.out_nbr_offsets[T + 1];
-    const std::uint32_t obs = b.slot_out_base[s];
-    for (std::uint32_t k = o0; k < o1; ++k) {
-      const std::uint32_t ns = find_slot(b, q, g.out_nbr_tiles[k]);
-      b.slot_out[obs + (k - o0)] = ns;
-      if (b.slot_out_off) b.slot_out_off[obs + (k - o0)] = ns == kNone ? ~0ull : b.slot_dist[ns];
+  if (lane == 0) {
+    b.stamp[s] = 0;  // also every queue-bit word of slot-order claims (ceil(S/32) <= S)
+    if (b.prio) b.prio[s] = kInfBits;
+  }
+  if (!structure) return;
+  const std::uint32_t q = b.slot_query[s], T = b.tiles[s];
+  const std::uint32_t in0 = g.in_nbr_offsets[T], in1 = g.in_nbr_offsets[T + 1];
+  const std::uint32_t o0 = g.out_nbr_offsets[T], o1 = g.out_nbr_offsets[T + 1];
+  const std::uint32_t in_base = b.slot_in_base[s], out_base = b.slot_out_base[s];
+  for (std::uint32_t k = lane; k < max(in1 - in0, o1 - o0); k += kSlotLanes) {
+    if (k < in1 - in0) b.slot_in[in_base + k] = find_slot(b, q, g.in_nbr_tiles[in0 + k]);
+    if (k < o1 - o0) {
+      const std::uint32_t ns = find_slot(b, q, g.out_nbr_tiles[o0 + k]);
+      b.slot_out[out_base + k] = ns;
+      if (b.slot_out_off) b.slot_out_off[out_base + k] = ns == kNone ? ~0ull : b.slot_dist[ns];
     }
   }
-  b.stamp[s] = 0;  // also every queue-bit word of slot-order claims (ceil(S/32) <= S)
-  if (b.prio) b.prio[s] = kInfBits;
-  // the relaxation kernel variant must hold the engine of every slot
-  const bool pull = b.engine[q] == kJacobiPull;
-  if (pull ? !holds_pull(b.engines) : !holds_push(b.engines))
-    atomicOr(&b.control->error_bits, 4u);
-  b.last_change[q] = 0;
-  if (structure && b.slot_desc) const_cast<SlotDesc*>(b.slot_desc)[s] = make_slot_desc(g, b, s);
+  if (lane == kSlotLanes - 1 && b.slot_desc) const_cast<SlotDesc*>(b.slot_desc)[s] = make_slot_desc(g, b, s);
 }
 
 // Zero the sources and queue round 0: Jacobi queues the source tiles and
-// every tile they feed; push engines queue the source tiles.
-__global__ void seed_kernel(DevGraph g, DevBatch b) {
-  const std::uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= b.query_count) return;
+// every tile they feed; push engines queue the source tiles.  One wave per
+// query; its lanes share the fed tiles of a source.
+__global__ __launch_bounds__(64) void seed_kernel(DevGraph g, DevBatch b) {
+  const std::uint32_t q = blockIdx.x, lane = threadIdx.x;
   const bool jacobi = b.engine[q] == kJacobiPull;
+  // the relaxation kernel variant must hold the engine of every query
+  if (lane == 0 && (jacobi ? !holds_pull(b.engines) : !holds_push(b.engines)))
+    atomicOr(&b.control->error_bits, 4u);
   for (std::uint32_t i = b.source_offsets[q]; i < b.source_offsets[q + 1]; ++i) {
     const std::uint32_t u = b.sources[i];
     const std::uint32_t T = g.owner_tiles[u];
     const std::uint32_t s = find_slot(b, q, T);
     if (s == kNone) {
-      atomicOr(&b.control->error_bits, 4u);  // device_failure: host validated this
+      if (lane == 0) atomicOr(&b.control->error_bits, 4u);  // device_failure: host validated this
       continue;
     }
-    const std::uint32_t v0 = g.tile_vertex_offsets[T];
-    const std::uint32_t npt = g.tile_vertex_offsets[T + 1] - v0;
-    std::uint32_t* column = b.dist + b.slot_dist[s];
-    column[u - v0] = 0u;
-    if (jacobi) column[npt + (u - v0)] = 0u;
-    if (b.prio && !jacobi) atomic_min_agent(&b.prio[s], 0u);
-    enqueue(b, s, 0);
+    if (lane == 0) {
+      const std::uint32_t v0 = g.tile_vertex_offsets[T];
+      const std::uint32_t npt = g.tile_vertex_offsets[T + 1] - v0;
+      std::uint32_t* column = b.dist + b.slot_dist[s];
+      column[u - v0] = 0u;
+      if (jacobi) column[npt + (u - v0)] = 0u;
+      if (b.prio && !jacobi) atomic_min_agent(&b.prio[s], 0u);
+      enqueue(b, s, 0);
+    }
     if (jacobi) {
       const std::uint32_t ob = b.slot_out_base[s];
       const std::uint32_t KO = g.out_nbr_offsets[T + 1] - g.out_nbr_offsets[T];
-      for (std::uint32_t k = 0; k < KO; ++k) {
+      for (std::uint32_t k = lane; k < KO; k += 64) {
         const std::uint32_t ns = b.slot_out[ob + k];
         if (ns != kNone) enqueue(b, ns, 0);
       }
@@ -231,8 +229,8 @@ __global__ void seed_kernel(DevGraph g, DevBatch b) {
   }
 }
 
-// Relaxation launch: the kernel variant of the batch's engine set, then
-// (one round per launch) the advance kernel.
+// Relaxation launch: the kernel variant of the batch's engine set, and for
+// slot-order claims the compaction between rounds.
 hipError_t relax_launch(std::uint32_t block, bool persistent, bool cooperative,
                         std::uint32_t grid, std::size_t lds_bytes, std::uint32_t max_v,
                         std::uint32_t work_words, const DevGraph& g, const DevBatch& b,
@@ -252,10 +250,7 @@ hipError_t relax_launch(std::uint32_t block, bool persistent, bool cooperative,
       e = relax_launch_mixed(block, persistent, cooperative, grid, lds_bytes, max_v, work_words, g, b, stream);
   }
   if (e != hipSuccess || persistent) return e;
-  if (b.ordered)
-    hipLaunchKernelGGL(ordered_advance_kernel, dim3(1), dim3(1024), 0, stream, b, 0u);
-  else
-    hipLaunchKernelGGL(relax_advance_kernel, dim3(1), dim3(64), 0, stream, b);
+  if (b.ordered) hipLaunchKernelGGL(ordered_advance_kernel, dim3(1), dim3(1024), 0, stream, b, 0u);
   return hipGetLastError();
 }
 
@@ -339,16 +334,14 @@ hipError_t coresident_per_cu(int device, int promised, std::uint32_t cus, std::s
 
 hipError_t prep_launch(const DevGraph& g, const DevBatch& b, std::uint64_t pool_words,
                        hipStream_t stream, bool structure) {
-  hipLaunchKernelGGL(reset_control_kernel, dim3(1), dim3(1024), 0, stream, b.control, b.queue, b.window);
-  const std::uint32_t fill_grid = 4096;
-  hipLaunchKernelGGL(fill_u32_kernel, dim3(fill_grid), dim3(256), 0, stream, b.dist,
-                     static_cast<unsigned long long>(pool_words), kInfBits);
-  if (b.slot_count)
-    hipLaunchKernelGGL(prep_slots_kernel, dim3((b.slot_count + 255) / 256), dim3(256), 0,
-                       stream, g, b, structure ? 1u : 0u);
-  if (b.query_count)
-    hipLaunchKernelGGL(seed_kernel, dim3((b.query_count + 127) / 128), dim3(128), 0, stream, g,
-                       b);
+  const std::uint32_t fill_blocks =
+      static_cast<std::uint32_t>(std::min<std::uint64_t>(4096, (pool_words + 4095) / 4096));
+  const std::uint32_t per_block = 256u / (structure ? kSlotLanes : 1u);
+  const std::uint32_t slot_blocks = (b.slot_count + per_block - 1) / per_block;
+  hipLaunchKernelGGL(prepare_kernel, dim3(fill_blocks + slot_blocks + 1), dim3(256), 0, stream, g, b,
+                     static_cast<unsigned long long>(pool_words), fill_blocks, slot_blocks,
+                     structure ? 1u : 0u);
+  if (b.query_count) hipLaunchKernelGGL(seed_kernel, dim3(b.query_count), dim3(64), 0, stream, g, b);
   if (b.ordered) hipLaunchKernelGGL(ordered_advance_kernel, dim3(1), dim3(1024), 0, stream, b, 1u);
   return hipGetLastError();
 }

@@ -866,9 +866,42 @@ __global__ __launch_bounds__(B, MW) void relax_persistent_kernel(DevGraph g, Dev
   }
 }
 
-// Host-polled control: one round per launch (ordinary grid), then the
-// advance kernel (jacobi_pull.hpp:153-220 shape: count the round, reset
-// the list that the next round fills, stop on an empty list or the limit).
+// After round r, by one wave (lane x looks after class x of the lists):
+// count the round, reset the list that the next round fills, stop on an
+// empty list or the round limit.
+__device__ __forceinline__ void advance_round(const DevBatch& b, std::uint32_t r) {
+  static_assert(kQueueClasses == 64, "one lane per class");
+  DevControl* c = b.control;
+  const std::uint32_t lane = threadIdx.x & 63u;
+  const bool any = __ballot(load_agent(list_count(b, (r + 1) % 3, lane)) != 0) != 0;
+  if (b.instrumentation) {
+    std::uint32_t n = load_agent(list_count(b, r % 3, lane));
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off);
+    if (lane == 0 && n > c->max_list) c->max_list = n;
+  }
+  store_agent(list_count(b, (r + 2) % 3, lane), 0u);
+  store_agent(list_claim(b, (r + 2) % 3, lane), 0u);
+  if (lane != 0) return;
+  if (b.prio) {
+    c->window_limit = next_window_limit(c, b, r, c->window_limit);
+    reset_next_min(c, (r + 2) % 3);
+  }
+  c->round = r + 1;
+  c->rounds_executed = r + 1;
+  if (!any) {
+    c->done = 1;
+    c->stop_reason = kStopConverged;
+  } else if (b.maximum_rounds && r + 1 >= b.maximum_rounds) {
+    c->done = 1;
+    c->stop_reason = kStopMaximumRounds;
+  }
+}
+
+// Host-polled control: one round per launch (ordinary grid); the workgroup
+// that finishes last advances the round (jacobi_pull.hpp:153-220 shape).  A
+// kernel of its own between the rounds cost 4.7 us and a launch gap per
+// round.  Workgroups arrive on group counters first, as at the persistent
+// grid's barrier: all on one counter would queue 11.4 ns each.
 template <int B, int EPT, bool I, int MW, int M>
 __global__ __launch_bounds__(B, MW) void relax_round_kernel(DevGraph g, DevBatch b,
                                                         std::uint32_t max_v,
@@ -882,11 +915,16 @@ __global__ __launch_bounds__(B, MW) void relax_round_kernel(DevGraph g, DevBatch
   if (!b.ordered && threadIdx.x < 64) queue = load_round_queue(b, r);
   const std::uint32_t limit = b.prio ? load_agent(&c->window_limit) : 0u;
   process_round<B, EPT, I, M>(g, b, r, queue, limit, l);
+  if (b.ordered) return;
+  __builtin_amdgcn_s_waitcnt(0);  // every wave's atomics of the round are performed
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  const bool last = threadIdx.x == 0 && arrive_last(c, gridDim.x);
+  if (__ballot(last)) advance_round(b, r);
 }
 
 // ---------------------------------------------------------------------------
-// Launch wrappers (host side; the advance kernel between round launches is
-// launched by relax.hip).
+// Launch wrappers (host side).
 // ---------------------------------------------------------------------------
 template <int B, int EPT, bool I, int MW, int M>
 hipError_t launch_relax(bool persistent, bool cooperative, std::uint32_t grid,

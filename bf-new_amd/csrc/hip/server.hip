@@ -164,14 +164,9 @@ __global__ void server_init_kernel(DevBatch b, std::uint32_t capacity, std::uint
     b.stamp[i] = 0;
   }
   if (i < kQueueWords / kBarrierStride) b.queue[i * kBarrierStride] = 0;
-  if (i == 0) {
-    DevControl* c = b.control;
-    c->round = 0;
-    c->done = 1;
-    c->stop_reason = 0;
-    c->error_bits = 0;
-    c->rounds_executed = 0;
-  }
+  // the whole control block at zero, and done until the first admission
+  if (i < sizeof(DevControl) / 4)
+    reinterpret_cast<std::uint32_t*>(b.control)[i] = i == offsetof(DevControl, done) / 4 ? 1u : 0u;
 }
 
 }  // namespace bfn
@@ -341,7 +336,7 @@ hipError_t bfn_server_s::step(std::uint32_t admit_count, std::uint32_t tile_coun
     if ((e = relax_launch(block, false, false, chunk_grid, lds_bytes, max_v, work_words, gview, view,
                           s)) != hipSuccess)
       return e;
-    launches += 2;
+    ++launches;
   }
   if ((e = fill_launch(d_done, 1, 0u, s)) != hipSuccess) return e;
   hipLaunchKernelGGL(harvest_kernel, dim3((Qcap + 255) / 256), dim3(256), 0, s, gview, view, Qcap,
@@ -614,7 +609,8 @@ int32_t bfn_server_create(bfn_device device, bfn_graph graph, const bfn_server_o
   b.pending = sv->d_pending;
   b.queue = sv->d_queue;
   b.control = sv->d_control;
-  const std::uint32_t n = std::max({sv->Scap, sv->Qcap + 1, kQueueWords / kBarrierStride});
+  const std::uint32_t n = std::max({sv->Scap, sv->Qcap + 1, kQueueWords / kBarrierStride,
+                                    static_cast<std::uint32_t>(sizeof(DevControl) / 4)});
   hipLaunchKernelGGL(server_init_kernel, dim3((n + 255) / 256), dim3(256), 0, sv->stream, b, sv->Qcap,
                      sv->Scap, sv->slab_words, sv->kin, sv->kout, sv->d_active, sv->d_src_off,
                      sv->d_tgt_off, sv->d_clean);
