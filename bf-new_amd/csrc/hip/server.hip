@@ -47,76 +47,106 @@ struct AdmitRecord {
   std::uint32_t pad;
 };
 
-// One block per admitted query.
-__global__ void admit_kernel(DevGraph g, DevBatch b, const AdmitRecord* records,
-                             const std::uint32_t* tiles, std::uint32_t* onpath,
-                             unsigned long long* frame_base, std::uint32_t* active,
-                             std::uint32_t slab_words, std::uint32_t kin, std::uint32_t kout) {
-  const AdmitRecord r = records[blockIdx.x];
-  const std::uint32_t tid = threadIdx.x;
+// Admission of a step's records, three launches over the admitted tiles
+// (flat index i = a record's tiles_offset + position): slot and query
+// records, then neighbour slots and cleared labels, then the sources.  (One
+// workgroup per query, a thread per slot with its 26 neighbour searches in
+// turn, took 634 us where a request selects all 4096 tiles.)
+constexpr std::uint32_t kAdmitLanes = 16;
+
+// The record of flat tile i: the last one whose tiles start at or before it.
+__device__ __forceinline__ AdmitRecord record_of(const AdmitRecord* records, std::uint32_t count,
+                                                 std::uint32_t i) {
+  std::uint32_t lo = 0, hi = count;
+  while (hi - lo > 1) {
+    const std::uint32_t mid = (lo + hi) >> 1;
+    if (records[mid].tiles_offset <= i) lo = mid; else hi = mid;
+  }
+  return records[lo];
+}
+
+__global__ void admit_tables_kernel(DevBatch b, const AdmitRecord* records, std::uint32_t count,
+                                    const std::uint32_t* tiles, std::uint32_t tile_count,
+                                    unsigned long long* frame_base, std::uint32_t* active,
+                                    std::uint32_t slab_words) {
+  const std::uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= tile_count) return;
+  const AdmitRecord r = record_of(records, count, i);
+  const std::uint32_t s = r.slot_begin + (i - r.tiles_offset);
+  const_cast<std::uint32_t*>(b.tiles)[s] = tiles[i];
+  const_cast<std::uint32_t*>(b.slot_query)[s] = r.query;
+  b.stamp[s] = 0;
+  if (i != r.tiles_offset) return;
   const std::uint32_t q = r.query;
-  for (std::uint32_t i = tid; i < r.slot_count; i += blockDim.x) {
-    const std::uint32_t s = r.slot_begin + i;
-    const_cast<std::uint32_t*>(b.tiles)[s] = tiles[r.tiles_offset + i];
-    const_cast<std::uint32_t*>(b.slot_query)[s] = q;
-    b.stamp[s] = 0;
+  const_cast<std::uint32_t*>(b.tile_begin)[q] = r.slot_begin;
+  const_cast<std::uint32_t*>(b.tile_end)[q] = r.slot_begin + r.slot_count;
+  const_cast<std::uint32_t*>(b.sources)[q] = r.source;
+  const_cast<std::uint32_t*>(b.targets)[q] = r.target;
+  const_cast<std::uint32_t*>(b.engine)[q] = r.engine;
+  b.last_change[q] = 0;
+  b.pending[q] = 0;
+  frame_base[q] = static_cast<unsigned long long>(r.slot_begin) * (slab_words / 2);
+  active[q] = 1;
+}
+
+__global__ __launch_bounds__(256) void admit_slots_kernel(DevGraph g, DevBatch b, const AdmitRecord* records,
+                                                          std::uint32_t count, std::uint32_t tile_count,
+                                                          std::uint32_t* onpath, std::uint32_t slab_words,
+                                                          std::uint32_t kin, std::uint32_t kout) {
+  const std::uint32_t i = blockIdx.x * (256u / kAdmitLanes) + threadIdx.x / kAdmitLanes;
+  const std::uint32_t lane = threadIdx.x % kAdmitLanes;
+  if (i >= tile_count) return;
+  const AdmitRecord r = record_of(records, count, i);
+  const std::uint32_t s = r.slot_begin + (i - r.tiles_offset);
+  const std::uint32_t T = b.tiles[s];
+  const std::uint32_t in0 = g.in_nbr_offsets[T], in1 = g.in_nbr_offsets[T + 1];
+  const std::uint32_t o0 = g.out_nbr_offsets[T], o1 = g.out_nbr_offsets[T + 1];
+  for (std::uint32_t k = lane; k < max(in1 - in0, o1 - o0); k += kAdmitLanes) {
+    if (k < in1 - in0)
+      b.slot_in[static_cast<std::size_t>(s) * kin + k] = find_slot(b, r.query, g.in_nbr_tiles[in0 + k]);
+    if (k < o1 - o0)
+      b.slot_out[static_cast<std::size_t>(s) * kout + k] = find_slot(b, r.query, g.out_nbr_tiles[o0 + k]);
   }
-  if (tid == 0) {
-    const_cast<std::uint32_t*>(b.tile_begin)[q] = r.slot_begin;
-    const_cast<std::uint32_t*>(b.tile_end)[q] = r.slot_begin + r.slot_count;
-    const_cast<std::uint32_t*>(b.sources)[q] = r.source;
-    const_cast<std::uint32_t*>(b.targets)[q] = r.target;
-    const_cast<std::uint32_t*>(b.engine)[q] = r.engine;
-    b.last_change[q] = 0;
-    b.pending[q] = 0;
-    frame_base[q] = static_cast<unsigned long long>(r.slot_begin) * (slab_words / 2);
-    active[q] = 1;
+  // a slot's slab is 2 max_v words: even, so pairs of words
+  uint2* labels = reinterpret_cast<uint2*>(b.dist + static_cast<std::size_t>(s) * slab_words);
+  uint2* marks = reinterpret_cast<uint2*>(onpath + static_cast<std::size_t>(s) * slab_words);
+  for (std::uint32_t w = lane; w < slab_words / 2; w += kAdmitLanes) {
+    labels[w] = make_uint2(kInfBits, kInfBits);
+    marks[w] = make_uint2(0u, 0u);
   }
-  __syncthreads();
-  const std::uint32_t qb = r.slot_begin, qe = r.slot_begin + r.slot_count;
-  for (std::uint32_t i = tid; i < r.slot_count; i += blockDim.x) {
-    const std::uint32_t s = r.slot_begin + i;
-    const std::uint32_t T = b.tiles[s];
-    const std::uint32_t in0 = g.in_nbr_offsets[T], in1 = g.in_nbr_offsets[T + 1];
-    for (std::uint32_t k = in0; k < in1; ++k)
-      b.slot_in[static_cast<std::size_t>(s) * kin + (k - in0)] = find_slot(b, q, g.in_nbr_tiles[k]);
-    const std::uint32_t o0 = g.out_nbr_offsets[T], o1 = g.out_nbr_offsets[T + 1];
-    for (std::uint32_t k = o0; k < o1; ++k)
-      b.slot_out[static_cast<std::size_t>(s) * kout + (k - o0)] = find_slot(b, q, g.out_nbr_tiles[k]);
+}
+
+// One wave per admitted query: its source's label and work for the round
+// that runs next.
+__global__ __launch_bounds__(64) void admit_seed_kernel(DevGraph g, DevBatch b, const AdmitRecord* records,
+                                                        std::uint32_t kout) {
+  const AdmitRecord r = records[blockIdx.x];
+  const std::uint32_t lane = threadIdx.x;
+  const std::uint32_t round = load_agent(&b.control->round);
+  const std::uint32_t u = r.source;
+  const std::uint32_t T = g.owner_tiles[u];
+  const std::uint32_t s = find_slot(b, r.query, T);
+  if (s == kNone) {
+    if (lane == 0) atomicOr(&b.control->error_bits, 4u);
+    return;
   }
-  const unsigned long long w0 = static_cast<unsigned long long>(qb) * slab_words;
-  const unsigned long long w1 = static_cast<unsigned long long>(qe) * slab_words;
-  for (unsigned long long w = w0 + tid; w < w1; w += blockDim.x) {
-    b.dist[w] = kInfBits;
-    onpath[w] = 0;
-  }
-  __syncthreads();
-  __threadfence();
-  if (tid == 0) {
-    const std::uint32_t round = load_agent(&b.control->round);
-    const std::uint32_t u = r.source;
-    const std::uint32_t T = g.owner_tiles[u];
-    const std::uint32_t s = find_slot(b, q, T);
-    if (s == kNone) {
-      atomicOr(&b.control->error_bits, 4u);
-      return;
-    }
+  const bool jacobi = r.engine == kJacobiPull;
+  if (lane == 0) {
     const std::uint32_t v0 = g.tile_vertex_offsets[T];
     const std::uint32_t npt = g.tile_vertex_offsets[T + 1] - v0;
     std::uint32_t* column = b.dist + b.slot_dist[s];
     column[u - v0] = 0u;
-    const bool jacobi = r.engine == kJacobiPull;
     if (jacobi) column[npt + (u - v0)] = 0u;
     enqueue(b, s, round);
-    b.pending[q] = round + 1;
-    if (jacobi) {
-      const std::uint32_t KO = g.out_nbr_offsets[T + 1] - g.out_nbr_offsets[T];
-      for (std::uint32_t k = 0; k < KO; ++k) {
-        const std::uint32_t ns = b.slot_out[static_cast<std::size_t>(s) * kout + k];
-        if (ns != kNone) enqueue(b, ns, round);
-      }
-    }
+    b.pending[r.query] = round + 1;
     store_agent(&b.control->done, 0u);
+  }
+  if (jacobi) {
+    const std::uint32_t KO = g.out_nbr_offsets[T + 1] - g.out_nbr_offsets[T];
+    for (std::uint32_t k = lane; k < KO; k += 64) {
+      const std::uint32_t ns = b.slot_out[static_cast<std::size_t>(s) * kout + k];
+      if (ns != kNone) enqueue(b, ns, round);
+    }
   }
 }
 
@@ -322,8 +352,12 @@ hipError_t bfn_server_s::step(std::uint32_t admit_count, std::uint32_t tile_coun
     if ((e = hipMemcpyAsync(d_upload_tiles, h_tiles, 4ull * tile_count, hipMemcpyHostToDevice,
                             s)) != hipSuccess)
       return e;
-    hipLaunchKernelGGL(admit_kernel, dim3(admit_count), dim3(256), 0, s, gview, view, d_records,
-                       d_upload_tiles, d_onpath, d_frame_base, d_active, slab_words, kin, kout);
+    hipLaunchKernelGGL(admit_tables_kernel, dim3((tile_count + 255) / 256), dim3(256), 0, s, view, d_records,
+                       admit_count, d_upload_tiles, tile_count, d_frame_base, d_active, slab_words);
+    const std::uint32_t per_block = 256u / kAdmitLanes;
+    hipLaunchKernelGGL(admit_slots_kernel, dim3((tile_count + per_block - 1) / per_block), dim3(256), 0, s,
+                       gview, view, d_records, admit_count, tile_count, d_onpath, slab_words, kin, kout);
+    hipLaunchKernelGGL(admit_seed_kernel, dim3(admit_count), dim3(64), 0, s, gview, view, d_records, kout);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   // No more workgroups than live slots (a round visits each at most once);
