@@ -125,7 +125,7 @@ struct bfn_graph_s {
   std::uint32_t V = 0, E = 0, T = 0, Rcsr = 0, Rcsc = 0;
   DeviceBuffer owner, tile_off, row_off, dst, w, row_runs, run_edges, run_dst, col_off, src, cw,
       eid, col_runs, crun_edges, crun_src, in_off, out_off, csc_pack, csr_pack, csc_rec, csr_rec,
-      csc_perm, csr_perm, csc_intra, csr_intra, csr_bnd, base_cost, occ_scratch, counts, stats;
+      csc_perm, csr_perm, csc_intra, csr_intra, csr_bnd, base_cost, next_cost, cost_scratch, occ_scratch, counts, stats;
   std::uint32_t* in_tiles = nullptr;
   std::uint32_t* in_stage = nullptr;
   std::uint32_t* out_tiles = nullptr;
@@ -581,18 +581,30 @@ int32_t bfn_graph_update_weights(bfn_graph graph, const float* csr_weights,
 
 namespace {
 int32_t apply_node_costs(bfn_graph graph, const float* base_cost, const int* device_occ) {
+  const std::size_t bytes = sizeof(float) * std::max(graph->V, 1u);
   if (base_cost) {
-    for (std::uint32_t v = 0; v < graph->V; ++v)
-      if (!(base_cost[v] >= 0.0f) || base_cost[v] > 3.4e38f)
-        return fail(BFN_E_INVALID_ARGUMENT, "node costs must be finite and nonnegative");
-    BFN_HIP(graph->base_cost.reserve(sizeof(float) * std::max(graph->V, 1u)));
-    BFN_HIP(hipMemcpyAsync(graph->base_cost.ptr, base_cost, sizeof(float) * graph->V,
+    // Checked on the device, in a buffer of their own: refused costs leave
+    // the last ones in place.  (The check on one host core took several
+    // milliseconds for 8.4M nodes.)
+    BFN_HIP(graph->next_cost.reserve(bytes));
+    BFN_HIP(hipMemcpyAsync(graph->next_cost.ptr, base_cost, sizeof(float) * graph->V,
                            hipMemcpyHostToDevice, graph->stream));
+    std::uint32_t* bad = graph->stats.as<std::uint32_t>() + 7;
+    std::uint32_t refused = 0;
+    BFN_HIP(fill_launch(bad, 1, 0u, graph->stream));
+    BFN_HIP(check_costs_launch(graph->next_cost.as<float>(), graph->V, bad, graph->stream));
+    BFN_HIP(hipMemcpyAsync(&refused, bad, sizeof refused, hipMemcpyDeviceToHost, graph->stream));
+    BFN_HIP(hipStreamSynchronize(graph->stream));
+    if (refused) return fail(BFN_E_INVALID_ARGUMENT, "node costs must be finite and nonnegative");
+    std::swap(graph->base_cost.ptr, graph->next_cost.ptr);
+    std::swap(graph->base_cost.capacity, graph->next_cost.capacity);
   } else if (!graph->base_cost.ptr) {
     return fail(BFN_E_STATE, "no base node costs uploaded yet");
   }
+  BFN_HIP(graph->cost_scratch.reserve(bytes));
   BFN_HIP(node_cost_launch(graph->view, graph->base_cost.as<float>(), device_occ,
-                           graph->w.as<float>(), graph->cw.as<float>(), graph->stream));
+                           graph->cost_scratch.as<float>(), graph->w.as<float>(), graph->cw.as<float>(),
+                           graph->stream));
   BFN_HIP(refresh_record_weights(graph->view, graph->csr_perm.as<std::uint32_t>(),
                                  graph->csc_perm.as<std::uint32_t>(), graph->stream));
   BFN_HIP(hipStreamSynchronize(graph->stream));
