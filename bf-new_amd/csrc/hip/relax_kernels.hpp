@@ -670,7 +670,7 @@ __device__ __forceinline__ std::uint32_t queued_slot(const DevBatch& b, const Ro
 template <int B, int EPT, bool I, int M>
 __device__ __forceinline__ void process_round(const DevGraph& g, const DevBatch& b, std::uint32_t r,
                               const RoundQueue& queue, std::uint32_t limit, const Lds& l) {
-  const std::uint32_t chunk = b.items_per_claim ? b.items_per_claim : 1u;
+  const std::uint32_t items = b.items_per_claim ? b.items_per_claim : 1u;
   VisitStats<I> st;
   std::uint32_t queued_min = kInfBits;
   if (threadIdx.x == 0) l.flags[4] = kInfBits;
@@ -721,7 +721,7 @@ __device__ __forceinline__ void process_round(const DevGraph& g, const DevBatch&
     std::uint32_t* seg_end = l.flags + 8;
     if (threadIdx.x == 0) {
       for (std::uint32_t x = 0; x < kBarrierGroups; ++x) seg_end[x] = c->seg_begin[x + 1];
-      ahead = atomic_add_agent(&c->seg_claim[home * kBarrierStride], chunk);
+      ahead = atomic_add_agent(&c->seg_claim[home * kBarrierStride], items);
     }
     for (;;) {
       if (threadIdx.x == 0) {
@@ -731,13 +731,13 @@ __device__ __forceinline__ void process_round(const DevGraph& g, const DevBatch&
           const std::uint32_t e = seg_end[y];
           if (ahead < e) {
             start = ahead;
-            end = min(ahead + chunk, e);
-            ahead = atomic_add_agent(&c->seg_claim[y * kBarrierStride], chunk);
+            end = min(ahead + items, e);
+            ahead = atomic_add_agent(&c->seg_claim[y * kBarrierStride], items);
             break;
           }
           if (++tried < kBarrierGroups)
             ahead = atomic_add_agent(&c->seg_claim[((home + tried) % kBarrierGroups) * kBarrierStride],
-                                     chunk);
+                                     items);
         }
         l.flags[0] = start;
         l.flags[2] = end;
@@ -757,7 +757,12 @@ __device__ __forceinline__ void process_round(const DevGraph& g, const DevBatch&
     // relaxation per batch: 32 point-Jacobi lanes on 32x32x128 580 -> 270 us,
     // 64 queries on 64x64x256 block Jacobi 2298 -> 1722 us and frontier push
     // 1240 -> 946 us, 256 queries on 128x128x512 15.1 -> 13.8 ms.
+    // A chunk is at most the list's share of a workgroup: with two items per
+    // claim, a round of fewer items than twice the grid left workgroups idle
+    // (64 queries on 64x64x256 935 -> 880 us, 256 on 128x128x512 13.61 ->
+    // 13.46 ms).
     const std::uint32_t li = r % 3;
+    const std::uint32_t chunk = max(1u, min(items, queue.n / gridDim.x));
     const std::uint32_t groups = min(gridDim.x, kQueueClasses);
     const std::uint32_t group = blockIdx.x % groups;
     const std::uint32_t dealt = group + groups * ((gridDim.x - group + groups - 1u) / groups);
