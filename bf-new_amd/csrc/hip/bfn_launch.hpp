@@ -129,11 +129,9 @@ hipError_t paths_launch(const PathArgs& a, std::uint32_t query_count, hipStream_
 hipError_t scan_u64_launch(const unsigned long long* in, unsigned long long* out, std::uint32_t n,
                            hipStream_t stream);
 hipError_t predecessors_launch(const DevGraph& g, const DevBatch& b, std::uint32_t q,
-                               std::uint32_t slots, std::uint32_t copy, std::uint32_t* out,
+                               std::uint32_t slots, std::uint32_t copy,
+                               const unsigned long long* offsets, std::uint32_t* out,
                                hipStream_t stream);
-hipError_t scatter_launch(const DevGraph& g, const DevBatch& b, std::uint32_t q,
-                          std::uint32_t slots, std::uint32_t copy, std::uint32_t* out,
-                          hipStream_t stream);
 hipError_t gather_region_launch(const DevGraph& g, const DevBatch& b, std::uint32_t q,
                                 std::uint32_t slots, std::uint32_t copy,
                                 const unsigned long long* offsets, std::uint32_t* out,

@@ -332,9 +332,11 @@ __global__ __launch_bounds__(512) void compact_paths_kernel(PathArgs a) {
   }
 }
 
-// Smallest-EdgeId tight admitted predecessor of each vertex of query q.
+// Smallest-EdgeId tight admitted predecessor of each vertex of query q, tile
+// by tile in the order of its sorted selected tiles (tile i at offsets[i]).
 __global__ void predecessors_kernel(DevGraph g, DevBatch b, std::uint32_t q,
-                                    std::uint32_t jacobi_copy, std::uint32_t* out) {
+                                    std::uint32_t jacobi_copy, const unsigned long long* offsets,
+                                    std::uint32_t* out) {
   const std::uint32_t pos = b.tile_begin[q] + blockIdx.x;
   if (pos >= b.tile_end[q]) return;
   const std::uint32_t s = slot_at(b, pos);
@@ -365,24 +367,9 @@ __global__ void predecessors_kernel(DevGraph g, DevBatch b, std::uint32_t q,
         }
       }
     }
-    out[v] = best_u;
+    out[offsets[blockIdx.x] + i] = best_u;
   }
 }
-
-// Scatters query q's final labels to global ids (out pre-filled with +inf).
-__global__ void scatter_distances_kernel(DevGraph g, DevBatch b, std::uint32_t q,
-                                         std::uint32_t jacobi_copy, std::uint32_t* out) {
-  const std::uint32_t pos = b.tile_begin[q] + blockIdx.x;
-  if (pos >= b.tile_end[q]) return;
-  const std::uint32_t s = slot_at(b, pos);
-  const std::uint32_t T = b.tiles[s];
-  const std::uint32_t v0 = g.tile_vertex_offsets[T];
-  const std::uint32_t npt = g.tile_vertex_offsets[T + 1] - v0;
-  const std::uint32_t* src =
-      b.dist + b.slot_dist[s] + static_cast<unsigned long long>(column_of(b, q, jacobi_copy)) * npt;
-  for (std::uint32_t i = threadIdx.x; i < npt; i += blockDim.x) out[v0 + i] = src[i];
-}
-
 
 __global__ void finalize_kernel(DevGraph g, DevBatch b, const unsigned long long* relaxations,
                                 QueryStatusDev* out, std::uint32_t* path_state) {
@@ -531,19 +518,11 @@ hipError_t scan_u64_launch(const unsigned long long* in, unsigned long long* out
 }
 
 hipError_t predecessors_launch(const DevGraph& g, const DevBatch& b, std::uint32_t q,
-                               std::uint32_t slots, std::uint32_t copy, std::uint32_t* out,
+                               std::uint32_t slots, std::uint32_t copy,
+                               const unsigned long long* offsets, std::uint32_t* out,
                                hipStream_t stream) {
   if (slots)
-    hipLaunchKernelGGL(predecessors_kernel, dim3(slots), dim3(256), 0, stream, g, b, q, copy, out);
-  return hipGetLastError();
-}
-
-hipError_t scatter_launch(const DevGraph& g, const DevBatch& b, std::uint32_t q,
-                          std::uint32_t slots, std::uint32_t copy, std::uint32_t* out,
-                          hipStream_t stream) {
-  if (slots)
-    hipLaunchKernelGGL(scatter_distances_kernel, dim3(slots), dim3(256), 0, stream, g, b, q, copy,
-                       out);
+    hipLaunchKernelGGL(predecessors_kernel, dim3(slots), dim3(256), 0, stream, g, b, q, copy, offsets, out);
   return hipGetLastError();
 }
 
