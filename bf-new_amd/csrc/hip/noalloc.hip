@@ -5,7 +5,8 @@
 // engines as bfn_batch_submit, with every piece of per-batch device state
 // (control block, batch description, slot tables, work lists, label pool,
 // per-query status, target labels) carved out of one file-scope static
-// device array, `scratch`, of kStaticScratchBytes per GPU.  The caller
+// device array, `scratch`, of kStaticScratchBytes per GPU; the counters of
+// the work lists have one of their own.  The caller
 // passes the batch (host arrays, copied in) and the host arrays the results
 // are copied out to.
 //

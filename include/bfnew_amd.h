@@ -346,8 +346,9 @@ int32_t bfn_batch_counters(bfn_workspace workspace, bfn_engine_counters *out);
  * forbid hipMalloc): the batch of bfn_batch_submit run to completion on the
  * graph's stream with no allocation at all.  Every piece of per-batch device
  * state lives in one static device array per GPU of
- * bfn_static_scratch_bytes() bytes (64 MiB), held until the process ends;
- * a batch that needs more returns BFN_E_OUT_OF_MEMORY before touching it.
+ * bfn_static_scratch_bytes() bytes (64 MiB) and the work-list counters in
+ * one of 48 KiB beside it, held until the process ends; a batch that needs
+ * more returns BFN_E_OUT_OF_MEMORY before touching them.
  * The batch is copied in from the caller's host arrays; per_query
  * ([query_count]) and target_distances ([target_offsets[query_count]],
  * +inf when unreached) are copied out before the call returns.  Tuning as
