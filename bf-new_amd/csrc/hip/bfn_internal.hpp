@@ -192,10 +192,7 @@ struct DevControl {
   alignas(128) std::uint32_t group_arrivals[kMaxArrivalGroups * kBarrierStride];
 };
 constexpr std::size_t kControlHead = offsetof(DevControl, barrier_count);
-// What workspace estimates and the static scratch count for a batch's control
-// block.
-constexpr std::size_t kControlBytes = 13312;
-static_assert(sizeof(DevControl) <= kControlBytes, "control block within its estimate");
+constexpr std::size_t kMinBufferBytes = 256;  // least size of a device allocation
 
 // What a visit of slot s needs before it can load any label: written once
 // per batch by the preparation kernel, so a visit starts with one 64-byte

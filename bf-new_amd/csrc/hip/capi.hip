@@ -55,7 +55,7 @@ struct DeviceBuffer {
   // Geometric growth, like DeviceBuffer::reserve (runtime.hip.cpp:222-240).
   hipError_t reserve(std::size_t bytes) {
     if (bytes <= capacity && ptr) return hipSuccess;
-    const std::size_t grown = std::max({bytes, std::size_t{256}, capacity + capacity / 2});
+    const std::size_t grown = std::max({bytes, kMinBufferBytes, capacity + capacity / 2});
     if (ptr) {
       (void)hipFree(ptr);
       ptr = nullptr;
@@ -833,11 +833,19 @@ std::size_t meta_layout(std::uint32_t Q, std::uint32_t S, std::uint32_t ns, std:
   return off;
 }
 
+// Device memory of a submit, buffer by buffer: description, neighbour slots
+// and their pool offsets, slot descriptors, queue stamps, window priorities,
+// work lists, labels, last changes, control block, list counters, status,
+// relaxation counts and path states.
 std::uint64_t batch_bytes(const BatchPlanHost& p, std::uint64_t meta_bytes) {
-  return meta_bytes + 4ull * (p.in_total + p.out_total) + 8ull * p.out_total +
-         (20ull + sizeof(SlotDesc)) * p.S +
-         4ull * p.pool_words + 4ull * p.Q * 2 + sizeof(QueryStatusDev) * p.Q + 8ull * p.Q +
-         kControlBytes;
+  const std::uint64_t S = p.S, Q = p.Q;
+  std::uint64_t total = 0;
+  for (const std::uint64_t n :
+       {meta_bytes, 4 * p.in_total, 4 * p.out_total, 8 * p.out_total, sizeof(SlotDesc) * S, 4 * S, 4 * S,
+        12 * S, 4 * p.pool_words, 4 * Q, std::uint64_t{sizeof(DevControl)}, std::uint64_t{4 * kQueueWords},
+        sizeof(QueryStatusDev) * Q, 8 * Q, 4 * Q})
+    total += std::max<std::uint64_t>(n, kMinBufferBytes);
+  return total;
 }
 
 // Sets up the DevBatch view over the workspace buffers.

@@ -203,7 +203,7 @@ int32_t bfn_batch_run_static(bfn_graph graph, const bfn_batch_desc* d, const bfn
     at = align256(at + std::max<std::size_t>(bytes, 4));
     return here;
   };
-  const std::size_t o_control = take(kControlBytes);
+  const std::size_t o_control = take(sizeof(DevControl));
   const std::size_t o_status = take(sizeof(QueryStatusDev) * Q);
   const std::size_t o_targets = take(4ull * nt);
   const std::size_t o_tile_off = take(4ull * (Q + 1));

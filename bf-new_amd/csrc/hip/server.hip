@@ -560,21 +560,25 @@ int32_t bfn_server_create(bfn_device device, bfn_graph graph, const bfn_server_o
   sv->block = o->block_size;
   sv->Qcap = o->max_active_queries;
   // bytes per tile slot: two label columns, path stamps, three frame words
-  // per vertex, neighbour tables, slot records and three list entries
+  // per vertex, neighbour tables, slot records, three list entries and the
+  // uploaded tile; per query: 13 words, path summary, length, offset and
+  // frame base, admission record; besides them the control block, the list
+  // counters and the least size of the 33 allocations
   const std::uint64_t per_slot = 4ull * sv->slab_words * 2 + 12ull * sv->max_v +
-                                 4ull * (sv->kin + sv->kout) + 40;
-  const std::uint64_t per_query = 4ull * 16 + 28;
+                                 4ull * (sv->kin + sv->kout) + 44;
+  const std::uint64_t per_query = 4ull * 13 + 28 + 3 * 8 + sizeof(AdmitRecord);
+  const std::uint64_t fixed = sizeof(DevControl) + 4ull * kQueueWords + 33ull * kMinBufferBytes;
   const std::uint64_t budget = o->budget_bytes ? o->budget_bytes : (1ull << 30);
-  if (budget <= per_query * sv->Qcap + per_slot)
+  if (budget <= fixed + per_query * sv->Qcap + per_slot)
     return bail(BFN_E_OUT_OF_MEMORY, "server budget holds no tile slots");
-  const std::uint64_t slots = (budget - per_query * sv->Qcap) / per_slot;
+  const std::uint64_t slots = (budget - fixed - per_query * sv->Qcap) / per_slot;
   sv->Scap = static_cast<std::uint32_t>(std::min<std::uint64_t>(slots, 0x7FFFFFFFull / sv->slab_words));
   sv->upload_tile_capacity = std::min<std::uint32_t>(sv->Scap, 1u << 22);
   if (hipStreamCreateWithFlags(&sv->stream, hipStreamNonBlocking) != hipSuccess)
     return bail(BFN_E_HIP, "stream creation failed");
   auto alloc = [&](auto** ptr, std::uint64_t bytes) {
     void* p = nullptr;
-    if (hipMalloc(&p, std::max<std::uint64_t>(bytes, 256)) != hipSuccess) return false;
+    if (hipMalloc(&p, std::max<std::uint64_t>(bytes, kMinBufferBytes)) != hipSuccess) return false;
     sv->allocations.push_back(p);
     *ptr = static_cast<std::remove_reference_t<decltype(*ptr)>>(p);
     return true;

@@ -265,7 +265,9 @@ int32_t bfn_graph_update_node_costs_from_workspace(bfn_graph graph,
                                                    const float *base_cost);
 
 /* Workspace (ReusableBatched*Workspace, batched_workspace.hpp; admission by
- * budget as estimate_batch_workspace, batch_workspace.cpp:163). */
+ * budget as estimate_batch_workspace, batch_workspace.cpp:163).  The budget
+ * and bfn_batch_estimate cover the device memory that a batch's submit takes
+ * in a new workspace; path, occupancy and image calls take theirs on top. */
 int32_t bfn_workspace_create(bfn_device device, uint64_t budget_bytes, bfn_workspace *out);
 int32_t bfn_workspace_free(bfn_workspace workspace);
 void bfn_tuning_default(bfn_tuning *out);

@@ -13,6 +13,9 @@
 // (fiber stack, default 256), EMU_TRACE (print every launch).
 #include "hip/hip_runtime.h"
 
+#include <map>
+#include <mutex>
+
 struct emu_event { std::chrono::steady_clock::time_point t; };
 struct emu_graph { std::vector<std::function<void()>> ops; };
 
@@ -178,6 +181,8 @@ emu_graph* end_capture() {
   return g;
 }
 
+std::uint64_t g_workgroups = 0;  // launched so far
+
 void launch(dim3 grid, dim3 block, std::size_t lds, bool concurrent, std::function<void()> body) {
   if (g_capturing) {
     g_capture->ops.push_back([=] { launch(grid, block, lds, concurrent, body); });
@@ -186,6 +191,7 @@ void launch(dim3 grid, dim3 block, std::size_t lds, bool concurrent, std::functi
   static const bool trace = std::getenv("EMU_TRACE") != nullptr;
   static std::uint64_t launches = 0;
   ++launches;
+  g_workgroups += grid.x;
   if (trace)
     std::fprintf(stderr, "[emu] launch %llu grid %u block %u lds %zu %s %s\n",
                  static_cast<unsigned long long>(launches), grid.x, block.x, lds,
@@ -233,14 +239,45 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) {
   return hipSuccess;
 }
 hipError_t hipDeviceSynchronize() { return hipSuccess; }
-hipError_t hipMalloc(void** p, std::size_t n) {
-  *p = std::aligned_alloc(256, (std::max<std::size_t>(n, 1) + 255) / 256 * 256);
-  if (*p) std::memset(*p, 0xCD, n);  // garbage, as device memory starts
-  return *p ? hipSuccess : hipErrorOutOfMemory;
+// Device (0) and pinned (1) memory in use, and the largest allocation of each
+// that is granted.
+namespace {
+std::mutex g_memory_mutex;
+std::map<void*, std::size_t> g_sizes[2];
+std::size_t g_used[2] = {0, 0}, g_largest[2] = {~std::size_t{0}, ~std::size_t{0}};
+hipError_t take_memory(int kind, void** p, std::size_t n) {
+  std::lock_guard<std::mutex> lock(g_memory_mutex);
+  *p = n > g_largest[kind] ? nullptr : std::aligned_alloc(256, (std::max<std::size_t>(n, 1) + 255) / 256 * 256);
+  if (!*p) return hipErrorOutOfMemory;
+  std::memset(*p, 0xCD, n);  // garbage, as device memory starts
+  g_sizes[kind][*p] = n;
+  g_used[kind] += n;
+  return hipSuccess;
 }
-hipError_t hipFree(void* p) { std::free(p); return hipSuccess; }
-hipError_t hipHostMalloc(void** p, std::size_t n, unsigned) { return hipMalloc(p, n); }
-hipError_t hipHostFree(void* p) { std::free(p); return hipSuccess; }
+hipError_t give_memory(int kind, void* p) {
+  std::lock_guard<std::mutex> lock(g_memory_mutex);
+  const auto it = g_sizes[kind].find(p);
+  if (it != g_sizes[kind].end()) {
+    g_used[kind] -= it->second;
+    g_sizes[kind].erase(it);
+  }
+  std::free(p);
+  return hipSuccess;
+}
+}  // namespace
+extern "C" std::uint64_t emu_memory_used(int kind) {
+  std::lock_guard<std::mutex> lock(g_memory_mutex);
+  return g_used[kind];
+}
+extern "C" void emu_largest_allocation(int kind, std::uint64_t bytes) {
+  std::lock_guard<std::mutex> lock(g_memory_mutex);
+  g_largest[kind] = bytes;
+}
+extern "C" std::uint64_t emu_workgroups() { return emu::g_workgroups; }
+hipError_t hipMalloc(void** p, std::size_t n) { return take_memory(0, p, n); }
+hipError_t hipFree(void* p) { return give_memory(0, p); }
+hipError_t hipHostMalloc(void** p, std::size_t n, unsigned) { return take_memory(1, p, n); }
+hipError_t hipHostFree(void* p) { return give_memory(1, p); }
 hipError_t hipMemcpyAsync(void* d, const void* s, std::size_t n, hipMemcpyKind, hipStream_t) {
   if (emu::capturing()) {
     emu::capture([=] { std::memcpy(d, s, n); });

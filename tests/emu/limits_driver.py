@@ -1,0 +1,93 @@
+"""Memory that the engine library named by argv[1] -- the CPU emulation of the
+kernels -- takes, against what it says it takes: the check argv[2], one JSON
+line on stdout with its failures."""
+import ctypes
+import json
+import os
+import sys
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+TESTS = os.path.dirname(HERE)
+ROOT = os.path.dirname(TESTS)
+sys.path.insert(0, os.path.join(ROOT, "bf-new_amd"))
+sys.path.insert(0, os.path.join(ROOT, "oracle"))
+sys.path.insert(0, TESTS)
+
+import numpy as np  # noqa: E402
+
+import bfnew_amd as bfn  # noqa: E402
+
+bfn.HIP_LIB_PATH = sys.argv[1]
+DEVICE, PINNED = 0, 1
+FAILURES = []
+
+
+def used(kind=DEVICE):
+    f = bfn.hip_lib().emu_memory_used
+    f.restype = ctypes.c_uint64
+    return f(kind)
+
+
+def check(ok, what):
+    if not ok:
+        FAILURES.append(what)
+
+
+def refused(f):
+    try:
+        f()
+    except bfn.BfnError as e:
+        return e.code
+    return 0
+
+
+def graph(dev, x=8, y=8, nodes=32):
+    hg = bfn.HostGraph.synthetic(x, y, nodes, 4, host_graph=True)
+    return hg, bfn.DeviceGraph(dev, hg.layout())
+
+
+def estimate(dev):
+    """A batch's estimate covers the device memory of its submit, and is the
+    smallest budget that admits it."""
+    hg, dg = graph(dev)
+    for count, engine, window in ((1, bfn.FRONTIER_PUSH, 0.0), (1, bfn.JACOBI_PULL, 0.0),
+                                  (9, bfn.FRONTIER_PUSH, 3.0)):
+        qs = hg.synthetic_queries(count, seed=5, side_min=2, side_max=4)
+        batch = bfn.Batch([[q.source] for q in qs], [[q.target] for q in qs],
+                          [hg.query_tiles(q) for q in qs])
+        o = bfn.run_options(engine=engine, control_mode=bfn.CHUNKED)
+        t = bfn.tuning(tile_sweeps=0, push_window=window)
+        before = used()
+        ws = bfn.Workspace(dev)
+        need = ws.estimate(dg, batch, o)
+        ws.submit(dg, batch, o, t)
+        check(used() - before <= need, f"batch of {count}: {used() - before} bytes in use, estimate {need}")
+        ws.close()
+        check(used() == before, "memory left after the workspace")
+        for budget, code in ((need, 0), (need - 1, 3)):
+            ws = bfn.Workspace(dev, budget)
+            got = refused(lambda: ws.submit(dg, batch, o, t))
+            check(got == code, f"batch of {count}, budget {budget} of {need}: {got}")
+            ws.close()
+
+
+def server(dev):
+    """A server's device memory stays within its budget."""
+    _, dg = graph(dev)
+    for budget, queries in ((256 << 10, 3), (1 << 20, 64), (8 << 20, 7)):
+        before = used()
+        s = bfn.Server(dev, dg, budget_bytes=budget, max_active_queries=queries)
+        check(used() - before <= budget, f"server: {used() - before} bytes in use of {budget}")
+        s.close()
+        check(used() == before, "memory left after the server")
+
+
+def main():
+    dev = bfn.Device(0)
+    globals()[sys.argv[2]](dev)
+    dev.close()
+    print(json.dumps(dict(check=sys.argv[2], failures=FAILURES)), flush=True)
+
+
+if __name__ == "__main__":
+    main()
