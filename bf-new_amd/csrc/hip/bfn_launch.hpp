@@ -143,7 +143,8 @@ hipError_t relaxation_count_launch(const DevGraph& g, const DevBatch& b,
                                    unsigned long long* out, hipStream_t stream);
 hipError_t occupancy_launch(const std::uint32_t* arena, unsigned long long n, int* occ,
                             hipStream_t stream);
-// cost: scratch of one float per vertex.
+// cost: scratch of one float per vertex, or null (the edges then read base
+// and occ).
 hipError_t node_cost_launch(const DevGraph& g, const float* base, const int* occ, float* cost,
                             float* csr_w, float* csc_w, hipStream_t stream);
 hipError_t check_costs_launch(const float* base, std::uint32_t n, std::uint32_t* bad, hipStream_t stream);

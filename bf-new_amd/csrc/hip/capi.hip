@@ -125,7 +125,7 @@ struct bfn_graph_s {
   std::uint32_t V = 0, E = 0, T = 0, Rcsr = 0, Rcsc = 0;
   DeviceBuffer owner, tile_off, row_off, dst, w, row_runs, run_edges, run_dst, col_off, src, cw,
       eid, col_runs, crun_edges, crun_src, in_off, out_off, csc_pack, csr_pack, csc_rec, csr_rec,
-      csc_perm, csr_perm, csc_intra, csr_intra, csr_bnd, base_cost, next_cost, cost_scratch, occ_scratch, counts, stats;
+      csc_perm, csr_perm, csc_intra, csr_intra, csr_bnd, base_cost, next_cost, occ_scratch, counts, stats;
   std::uint32_t* in_tiles = nullptr;
   std::uint32_t* in_stage = nullptr;
   std::uint32_t* out_tiles = nullptr;
@@ -580,31 +580,58 @@ int32_t bfn_graph_update_weights(bfn_graph graph, const float* csr_weights,
 }
 
 namespace {
+// Up to this many vertices new node costs are checked on the host and the
+// edge weights computed from costs and occupancy in one launch; beyond it the
+// check runs on the device and, with an occupancy, a pass writes each node's
+// cost once for the edges to read.  Update with new costs, host against
+// device check: 65k vertices 55 / 74 us, 262k 131 / 131, 501k 207 / 180.
+// Update from a workspace's occupancy, one launch against the pass: 65k 43 /
+// 46 us, 262k 67 / 67, 501k 101 / 92, 8.4M 1772 / 1379.
+constexpr std::uint32_t kSmallGraphVertices = 1u << 18;
+
 int32_t apply_node_costs(bfn_graph graph, const float* base_cost, const int* device_occ) {
-  const std::size_t bytes = sizeof(float) * std::max(graph->V, 1u);
+  const std::uint32_t V = graph->V;
+  const std::size_t bytes = sizeof(float) * std::max(V, 1u);
+  // A second buffer of the costs' size, where there is memory for it: new
+  // costs are staged there until they are checked (refused costs leave the
+  // last ones in place), then it holds the nodes' costs.
+  auto second_buffer = [&] {
+    if (V <= kSmallGraphVertices) return false;
+    const bool there = graph->next_cost.reserve(bytes) == hipSuccess;
+    if (!there) (void)hipGetLastError();
+    return there;
+  };
   if (base_cost) {
-    // Checked on the device, in a buffer of their own: refused costs leave
-    // the last ones in place.  (The check on one host core took several
-    // milliseconds for 8.4M nodes.)
-    BFN_HIP(graph->next_cost.reserve(bytes));
-    BFN_HIP(hipMemcpyAsync(graph->next_cost.ptr, base_cost, sizeof(float) * graph->V,
-                           hipMemcpyHostToDevice, graph->stream));
-    std::uint32_t* bad = graph->stats.as<std::uint32_t>() + 7;
-    std::uint32_t refused = 0;
-    BFN_HIP(fill_launch(bad, 1, 0u, graph->stream));
-    BFN_HIP(check_costs_launch(graph->next_cost.as<float>(), graph->V, bad, graph->stream));
-    BFN_HIP(hipMemcpyAsync(&refused, bad, sizeof refused, hipMemcpyDeviceToHost, graph->stream));
-    BFN_HIP(hipStreamSynchronize(graph->stream));
-    if (refused) return fail(BFN_E_INVALID_ARGUMENT, "node costs must be finite and nonnegative");
-    std::swap(graph->base_cost.ptr, graph->next_cost.ptr);
-    std::swap(graph->base_cost.capacity, graph->next_cost.capacity);
+    const bool staged = second_buffer();
+    bool fine = true;
+    if (staged) {
+      std::uint32_t* bad = graph->stats.as<std::uint32_t>() + 7;
+      std::uint32_t refused = 0;
+      BFN_HIP(hipMemcpyAsync(graph->next_cost.ptr, base_cost, sizeof(float) * V, hipMemcpyHostToDevice,
+                             graph->stream));
+      BFN_HIP(fill_launch(bad, 1, 0u, graph->stream));
+      BFN_HIP(check_costs_launch(graph->next_cost.as<float>(), V, bad, graph->stream));
+      BFN_HIP(hipMemcpyAsync(&refused, bad, sizeof refused, hipMemcpyDeviceToHost, graph->stream));
+      BFN_HIP(hipStreamSynchronize(graph->stream));
+      fine = refused == 0;
+    } else {
+      for (std::uint32_t v = 0; v < V; ++v) fine &= base_cost[v] >= 0.0f && base_cost[v] <= 3.4e38f;
+    }
+    if (!fine) return fail(BFN_E_INVALID_ARGUMENT, "node costs must be finite and nonnegative");
+    if (staged) {
+      std::swap(graph->base_cost.ptr, graph->next_cost.ptr);
+      std::swap(graph->base_cost.capacity, graph->next_cost.capacity);
+    } else {
+      BFN_HIP(graph->base_cost.reserve(bytes));
+      BFN_HIP(hipMemcpyAsync(graph->base_cost.ptr, base_cost, sizeof(float) * V, hipMemcpyHostToDevice,
+                             graph->stream));
+    }
   } else if (!graph->base_cost.ptr) {
     return fail(BFN_E_STATE, "no base node costs uploaded yet");
   }
-  BFN_HIP(graph->cost_scratch.reserve(bytes));
-  BFN_HIP(node_cost_launch(graph->view, graph->base_cost.as<float>(), device_occ,
-                           graph->cost_scratch.as<float>(), graph->w.as<float>(), graph->cw.as<float>(),
-                           graph->stream));
+  float* cost = device_occ && second_buffer() ? graph->next_cost.as<float>() : nullptr;
+  BFN_HIP(node_cost_launch(graph->view, graph->base_cost.as<float>(), device_occ, cost, graph->w.as<float>(),
+                           graph->cw.as<float>(), graph->stream));
   BFN_HIP(refresh_record_weights(graph->view, graph->csr_perm.as<std::uint32_t>(),
                                  graph->csc_perm.as<std::uint32_t>(), graph->stream));
   BFN_HIP(hipStreamSynchronize(graph->stream));

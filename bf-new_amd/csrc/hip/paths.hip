@@ -26,6 +26,8 @@
 // candidates in exactly the reference's cursor order.
 #include "bfn_internal.hpp"
 
+#include <algorithm>
+
 namespace bfn {
 
 
@@ -428,43 +430,47 @@ __global__ void occupancy_kernel(const std::uint32_t* arena_vertices, unsigned l
     atomicAdd(&occupancy[arena_vertices[i]], 1);
 }
 
-// w(u -> v) = base[v] * (1 + 0.5 * occ[v]) in this fp32 order, once per node.
-__global__ void node_cost_kernel(const float* base, const int* occupancy, std::uint32_t n, float* cost) {
-  const std::uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= n) return;
+// w(u -> v) = base[v] * (1 + 0.5 * occ[v]) in this fp32 order.
+__device__ __forceinline__ float node_cost(const float* base, const int* occupancy, std::uint32_t v) {
   const float occ = occupancy ? static_cast<float>(occupancy[v]) : 0.0f;
   const float scale = 1.0f + 0.5f * occ;
-  cost[v] = base[v] * scale;
+  return base[v] * scale;
 }
 
-// The weights of both orientations from the node costs, one thread per edge
-// so that the arrays are written in whole lines.  (One thread per node wrote
+__global__ void node_cost_kernel(const float* base, const int* occupancy, std::uint32_t n, float* cost) {
+  const std::uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
+  if (v < n) cost[v] = node_cost(base, occupancy, v);
+}
+
+// The weights of both orientations, one thread per edge so that the arrays
+// are written in whole lines: the first `csr_blocks` workgroups take the CSR
+// edges (their destination's cost), the others 256 columns of the CSC each
+// (found by a search of their offsets in LDS).  (One thread per node wrote
 // ten edges apart from its neighbours' and read two arrays per edge: 1137 us
-// for 84M edges.)  CSR: the destination's cost.  CSC: the column's cost; a
-// workgroup's 256 columns are found by a search of their offsets in LDS.
-__global__ __launch_bounds__(256) void csr_cost_kernel(const std::uint32_t* destinations, const float* cost,
-                                                       std::uint32_t n, float* weights) {
-  const std::uint32_t stride = gridDim.x * 256u;
-  for (unsigned long long e = blockIdx.x * 256u + threadIdx.x; e < n; e += stride)
-    weights[e] = cost[destinations[e]];
-}
-
-__global__ __launch_bounds__(256) void csc_cost_kernel(const std::uint32_t* offsets, const float* cost,
-                                                       std::uint32_t n, float* weights) {
+// for 84M edges.)
+__global__ __launch_bounds__(256) void edge_cost_kernel(DevGraph g, const float* base, const int* occupancy,
+                                                        std::uint32_t csr_blocks, float* csr_weights,
+                                                        float* csc_weights) {
+  const std::uint32_t tid = threadIdx.x;
+  if (blockIdx.x < csr_blocks) {
+    for (unsigned long long e = blockIdx.x * 256ull + tid; e < g.edge_count; e += csr_blocks * 256ull)
+      csr_weights[e] = node_cost(base, occupancy, g.destinations[e]);
+    return;
+  }
   __shared__ std::uint32_t ends[256];
   __shared__ float costs[256];
-  const std::uint32_t v0 = blockIdx.x * 256u, tid = threadIdx.x;
-  const std::uint32_t count = min(256u, n - v0);
-  const std::uint32_t begin = offsets[v0], end = offsets[v0 + count];
-  ends[tid] = tid < count ? offsets[v0 + tid + 1] : end;
-  costs[tid] = tid < count ? cost[v0 + tid] : 0.0f;
+  const std::uint32_t v0 = (blockIdx.x - csr_blocks) * 256u;
+  const std::uint32_t count = min(256u, g.vertex_count - v0);
+  const std::uint32_t begin = g.column_offsets[v0], end = g.column_offsets[v0 + count];
+  ends[tid] = tid < count ? g.column_offsets[v0 + tid + 1] : end;
+  costs[tid] = tid < count ? node_cost(base, occupancy, v0 + tid) : 0.0f;
   __syncthreads();
   for (unsigned long long e = static_cast<unsigned long long>(begin) + tid; e < end; e += 256) {
     std::uint32_t c = 0;  // columns that end at or before e
 #pragma unroll
     for (std::uint32_t step = 128; step > 0; step >>= 1)
       if (ends[c + step - 1] <= e) c += step;
-    weights[e] = costs[c];
+    csc_weights[e] = costs[c];
   }
 }
 
@@ -577,18 +583,18 @@ hipError_t occupancy_launch(const std::uint32_t* arena, unsigned long long n, in
 
 hipError_t node_cost_launch(const DevGraph& g, const float* base, const int* occ, float* cost,
                             float* csr_w, float* csc_w, hipStream_t stream) {
-  const std::uint32_t V = g.vertex_count;
+  const std::uint32_t V = g.vertex_count, columns = (V + 255u) / 256u;
   if (V == 0) return hipSuccess;
-  hipLaunchKernelGGL(node_cost_kernel, dim3((V + 255) / 256), dim3(256), 0, stream, base, occ, V, cost);
-  hipLaunchKernelGGL(csr_cost_kernel, dim3(8192), dim3(256), 0, stream, g.destinations, cost, g.edge_count,
-                     csr_w);
-  hipLaunchKernelGGL(csc_cost_kernel, dim3((V + 255) / 256), dim3(256), 0, stream, g.column_offsets, cost, V,
-                     csc_w);
+  if (cost) hipLaunchKernelGGL(node_cost_kernel, dim3(columns), dim3(256), 0, stream, base, occ, V, cost);
+  const std::uint32_t csr_blocks = std::min(8192u, (g.edge_count + 255u) / 256u);
+  hipLaunchKernelGGL(edge_cost_kernel, dim3(csr_blocks + columns), dim3(256), 0, stream, g, cost ? cost : base,
+                     cost ? nullptr : occ, csr_blocks, csr_w, csc_w);
   return hipGetLastError();
 }
 
 hipError_t check_costs_launch(const float* base, std::uint32_t n, std::uint32_t* bad, hipStream_t stream) {
-  hipLaunchKernelGGL(check_costs_kernel, dim3(1024), dim3(256), 0, stream, base, n, bad);
+  hipLaunchKernelGGL(check_costs_kernel, dim3(std::min(1024u, (n + 255u) / 256u)), dim3(256), 0, stream, base,
+                     n, bad);
   return hipGetLastError();
 }
 

@@ -18,6 +18,9 @@ import numpy as np  # noqa: E402
 import bfnew_amd as bfn  # noqa: E402
 
 bfn.HIP_LIB_PATH = sys.argv[1]
+
+from helpers import bits, oracle_query  # noqa: E402
+
 DEVICE, PINNED = 0, 1
 FAILURES = []
 
@@ -80,6 +83,65 @@ def server(dev):
         check(used() - before <= budget, f"server: {used() - before} bytes in use of {budget}")
         s.close()
         check(used() == before, "memory left after the server")
+
+
+def largest(kind, n_bytes):
+    bfn.hip_lib().emu_largest_allocation(kind, ctypes.c_uint64(n_bytes))
+
+
+def workgroups():
+    f = bfn.hip_lib().emu_workgroups
+    f.restype = ctypes.c_uint64
+    return f()
+
+
+def expect_weights(dev, dg, view, costs):
+    """Labels of one region under both weight orientations against the oracle."""
+    tiles = np.arange(9, dtype=np.uint32)
+    view["weights"] = costs[view["destinations"]]
+    want, _ = oracle_query(view, [5], tiles)
+    for engine in (bfn.JACOBI_PULL, bfn.FRONTIER_PUSH):
+        ws = bfn.Workspace(dev)
+        ws.submit(dg, bfn.Batch([[5]], [[100]], [tiles]),
+                  bfn.run_options(engine=engine, control_mode=bfn.CHUNKED), bfn.tuning(tile_sweeps=0))
+        check(np.array_equal(bits(ws.distances(0)), bits(want)), f"labels under engine {engine}")
+        ws.close()
+
+
+def costs(dev):
+    """Node-cost updates: what they keep (the costs and the occupancy; on a
+    large graph a second buffer where there is memory for it, and the update
+    as before where there is none), and the workgroups of a small graph's."""
+    half = np.float32(0.5)
+    for dims, extra in (((16, 16, 33), 0), ((32, 32, 257), 1)):
+        hg, dg = graph(dev, *dims)
+        view = hg.view()
+        V = view["vertex_count"]
+        base = np.random.default_rng(V).uniform(0.5, 9.0, V).astype(np.float32)
+        occupancy = (np.arange(V) % 3).astype(np.int32)
+        before, at = used(), workgroups()
+        dg.update_node_costs(base)
+        groups = workgroups() - at
+        blocks = -(-view["edge_count"] // 256)
+        check(extra or groups <= 4 * blocks, f"{groups} workgroups for {view['edge_count']} edges")
+        dg.update_node_costs(base * half)
+        dg.update_node_costs(base, occupancy)
+        kept = used() - before
+        check(kept <= 4 * V * (2 + extra), f"{kept} bytes kept for {V} vertices")
+        expect_weights(dev, dg, view, base * (np.float32(1.0) + half * occupancy.astype(np.float32)))
+        bad = base.copy()
+        bad[V - 1] = np.nan
+        check(refused(lambda: dg.update_node_costs(bad)) == 1, "NaN costs accepted")
+        dg.close()
+    # no memory for more than the costs
+    hg, dg = graph(dev, 32, 32, 257)
+    dg.update_node_costs(base)
+    largest(DEVICE, 0)
+    check(refused(lambda: dg.update_node_costs(base + half)) == 0, "update without a second buffer")
+    check(refused(lambda: dg.update_node_costs(bad)) == 1, "NaN costs accepted")
+    largest(DEVICE, 1 << 40)
+    expect_weights(dev, dg, view, base + half)
+    dg.close()
 
 
 def main():

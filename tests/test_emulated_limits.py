@@ -1,6 +1,7 @@
 """Device and pinned memory of the engine library, counted allocation by
 allocation on the CPU emulation of the kernels (tests/emu): estimates and
-budgets against what is allocated.  Each check of tests/emu/limits_driver.py
+budgets against what is allocated, and calls that are to work where memory for
+their faster form is missing.  Each check of tests/emu/limits_driver.py
 runs in a process of its own, since it loads the emulated library."""
 import json
 import os
@@ -15,7 +16,7 @@ sys.path.insert(0, os.path.join(HERE, "emu"))
 import build_emu  # noqa: E402
 
 
-@pytest.mark.parametrize("check", ["estimate", "server"])
+@pytest.mark.parametrize("check", ["estimate", "server", "costs"])
 def test_emulated_limits(check):
     lib = build_emu.build()
     env = dict(os.environ)

@@ -1,4 +1,5 @@
-"""Node costs on a vertex count that is no multiple of the kernels' blocks:
+"""Node costs on vertex counts that are no multiple of the kernels' blocks,
+on both sides of the size up to which costs are checked on the host:
 the weights of both orientations against the oracle, and refused costs
 (negative, infinite, NaN) leaving the last accepted ones in place."""
 import numpy as np
@@ -10,8 +11,9 @@ from helpers import bits, oracle_query
 pytestmark = pytest.mark.gpu
 
 
-def test_refused_costs_leave_the_last_ones(device):
-    hg = bfn.HostGraph.synthetic(9, 8, 33, 3, host_graph=True)
+@pytest.mark.parametrize("dims", [(9, 8, 33), (32, 32, 257)])
+def test_refused_costs_leave_the_last_ones(device, dims):
+    hg = bfn.HostGraph.synthetic(*dims, 3, host_graph=True)
     view = hg.view()
     dg = bfn.DeviceGraph(device, hg.layout())
     costs = np.random.default_rng(1).uniform(0.5, 9.0, view["vertex_count"]).astype(np.float32)
