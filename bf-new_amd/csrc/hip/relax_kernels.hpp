@@ -148,6 +148,25 @@ struct VisitStats {
   }
 };
 
+// Whether the workgroup takes a visit's slabs one after the other, four
+// words per thread in flight, rather than `Slabs` slabs per wave and `Rows`
+// 64-word rows of each: the form with fewer round trips (slabs are taken to
+// be of the visited tile's size).  It is the one for large tiles with few
+// neighbours, where most waves would have no slab.  Relaxation of 24 queries,
+// slabs per wave / one after the other: point Jacobi on one tile of 4000
+// vertices, 256 threads 421 / 316 us, 1024 threads 293 / 181; dense push
+// through proposals on two tiles of 2000, 1024 threads 265 / 221; on 3x3
+// tiles of 2000, 1024 threads 382 / 332.
+template <int B, std::uint32_t Slabs, std::uint32_t Rows>
+__device__ __forceinline__ bool slab_by_slab(std::uint32_t slabs, std::uint32_t words) {
+  constexpr std::uint32_t kAtOnce = Slabs * (B / 64);
+  // uniform values, said to be so: a branch on them without it cost 2 %
+  slabs = __builtin_amdgcn_readfirstlane(slabs);
+  words = __builtin_amdgcn_readfirstlane(words);
+  return slabs * ((words + 4 * B - 1) / (4 * B)) <
+         (words + 64 * Rows - 1) / (64 * Rows) * ((slabs + kAtOnce - 1) / kAtOnce);
+}
+
 __device__ __forceinline__ std::uint32_t pk_k(std::uint32_t p) { return p >> 24; }
 __device__ __forceinline__ std::uint32_t pk_src(std::uint32_t p) { return (p >> 12) & kPackLocalMask; }
 __device__ __forceinline__ std::uint32_t pk_dst(std::uint32_t p) { return p & kPackLocalMask; }
@@ -201,7 +220,26 @@ __device__ __forceinline__ void visit_pull(const DevGraph& g, const DevBatch& b,
   // flight, so a list of up to 16 small slabs costs one round trip.
   constexpr std::uint32_t kSlabs = 4, kRows = 2, kWaves = B / 64;
   const std::uint32_t lane = tid & 63u, wave = tid >> 6;
-  for (std::uint32_t k0 = wave; k0 < K; k0 += kSlabs * kWaves) {
+  const bool one_by_one = slab_by_slab<B, kSlabs, kRows>(K, npt);
+  for (std::uint32_t k = one_by_one ? 0u : K; k < K; ++k) {
+    const std::uint32_t n = l.marks[k], at = l.slots[k], hi = l.offs[2 * k + 1];
+    const std::uint32_t* src = b.dist + ((static_cast<unsigned long long>(hi) << 32) | l.offs[2 * k]);
+    for (std::uint32_t i0 = tid; i0 < n; i0 += 4 * B) {
+      std::uint32_t x[4];
+#pragma unroll
+      for (std::uint32_t r = 0; r < 4; ++r) {
+        x[r] = kInfBits;
+        if (hi != kNone && i0 + r * B < n) x[r] = src[i0 + r * B];
+      }
+#pragma unroll
+      for (std::uint32_t r = 0; r < 4; ++r)
+        if (i0 + r * B < n) {
+          l.work[at + i0 + r * B] = x[r];
+          if (k == 0) l.own[i0 + r * B] = x[r];
+        }
+    }
+  }
+  for (std::uint32_t k0 = one_by_one ? K : wave; k0 < K; k0 += kSlabs * kWaves) {
     const std::uint32_t* src[kSlabs];
     std::uint32_t size[kSlabs], at[kSlabs], longest = 0;
 #pragma unroll
@@ -471,7 +509,31 @@ __device__ __forceinline__ void visit_push(const DevGraph& g, const DevBatch& b,
     // 45x37x301 tiles, relaxation 903 -> 545 us.)
     constexpr std::uint32_t kSlabs = 2, kRows = 4, kWaves = B / 64;
     const std::uint32_t lane = tid & 63u, wave = tid >> 6;
-    for (std::uint32_t k0 = 1 + wave; k0 < KO; k0 += kSlabs * kWaves) {
+    const bool one_by_one = slab_by_slab<B, kSlabs, kRows>(KO - 1, npt);
+    for (std::uint32_t k = one_by_one ? 1u : KO; k < KO; ++k) {
+      const std::uint32_t ns = l.slots[k], at = l.offs[k] & 0xFFFFu, n = l.offs[k] >> 16;
+      if (ns == kNone) continue;
+      std::uint32_t* target = b.dist + (b.slot_out_off ? b.slot_out_off[out_base + k] : b.slot_dist[ns]);
+      if (tid == 0) st.bytes += 4ull * n;  // the neighbour slab, read once
+      std::uint32_t low = kInfBits;
+      for (std::uint32_t i0 = tid; i0 < n; i0 += 4 * B) {
+        std::uint32_t seen[4];
+#pragma unroll
+        for (std::uint32_t r4 = 0; r4 < 4; ++r4) seen[r4] = i0 + r4 * B < n ? target[i0 + r4 * B] : 0u;
+#pragma unroll
+        for (std::uint32_t r4 = 0; r4 < 4; ++r4) {
+          if (i0 + r4 * B >= n) continue;
+          const std::uint32_t pv = l.prop[at + i0 + r4 * B];
+          if (pv < seen[r4]) {
+            atomic_min_agent(target + i0 + r4 * B, pv);
+            ++suc;
+            low = min(low, pv);
+          }
+        }
+      }
+      if (low != kInfBits) atomicMin(&l.marks[k], low);
+    }
+    for (std::uint32_t k0 = one_by_one ? KO : 1 + wave; k0 < KO; k0 += kSlabs * kWaves) {
       std::uint32_t* target[kSlabs];
       std::uint32_t size[kSlabs], at[kSlabs], low[kSlabs], longest = 0;
 #pragma unroll

@@ -1,6 +1,6 @@
 """Every engine and control mode on tile sizes at the edges of what a visit
-stages at a time (64-word rows, four rows per slab, the registers that hold a
-tile's internal records), against the oracle bit for bit.  The 9 x 8 grid
+stages at a time (64-word rows, two of a pulled slab and four of a proposal slab
+together, the registers that hold a tile's internal records), against the oracle bit for bit.  The 9 x 8 grid
 clamps its long edges, so tiles have between 5 and 13 neighbours, and the
 boxes leave some of them out; the batches have fewer slots than work-list
 classes and more, and claims of several items."""
@@ -20,6 +20,39 @@ CONFIGS = [
     dict(engine=bfn.FRONTIER_PUSH, control=bfn.CHUNKED, sweeps=0, boundary=1, window=4.0,
          per_claim=5),
 ]
+
+
+def check_grid(device, dims, block):
+    hg = bfn.HostGraph.synthetic(*dims, 7, host_graph=True)
+    view = hg.view()
+    dg = bfn.DeviceGraph(device, hg.layout())
+    rng = np.random.default_rng(dims[2])
+    ends = rng.integers(0, view["vertex_count"], (7, 2))
+    tiles = np.arange(dims[0] * dims[1], dtype=np.uint32)
+    batch = bfn.Batch([[int(s)] for s, _ in ends], [[int(t)] for _, t in ends], [tiles] * 7)
+    want = [oracle_query(view, [int(s)], tiles)[0] for s, _ in ends]
+    for c in CONFIGS:
+        print("grid", dims, block, c, flush=True)
+        ws = bfn.Workspace(device)
+        ws.submit(dg, batch, bfn.run_options(engine=c["engine"], control_mode=c["control"],
+                                             rounds_per_chunk=3, block_size=block),
+                  bfn.tuning(tile_sweeps=c["sweeps"], boundary_mode=c["boundary"],
+                             push_window=c.get("window", 0.0),
+                             items_per_claim=c.get("per_claim", 1)))
+        assert ws.status()[0].converged == 1, c
+        for i in range(len(ends)):
+            assert np.array_equal(bits(ws.distances(i)), bits(want[i])), (c, i)
+        ws.close()
+    dg.close()
+
+
+@pytest.mark.parametrize("dims,block", [((1, 1, 130), 64), ((2, 1, 257), 64), ((1, 1, 2049), 512),
+                                        ((2, 1, 1023), 256), ((4, 1, 1025), 256),
+                                        ((3, 3, 2000), 1024)])
+def test_few_large_tiles_bit_exact(device, dims, block):
+    """Grids of few tiles, whose slabs the whole workgroup takes one by one:
+    sizes about its four words per thread."""
+    check_grid(device, dims, block)
 
 
 @pytest.mark.parametrize("nodes,block", [(1, 64), (2, 256), (63, 64), (64, 128), (65, 256),
