@@ -1282,11 +1282,18 @@ namespace {
 
 // One query's image over its selected tiles (labels, or predecessors), tile
 // by tile in their sorted order: computed on the device and copied to pinned
-// memory.  offsets[i] is where tile i starts, the last entry the total.
-int32_t region_image(bfn_workspace ws, std::uint32_t query, bool predecessors,
-                     std::vector<unsigned long long>& offsets, const std::uint32_t** image) {
+// memory (or, where there is none, to `plain`).  offsets[i] is where tile i
+// starts, the last entry the total.
+struct RegionImage {
+  std::vector<unsigned long long> offsets;
+  std::vector<std::uint32_t> plain;
+  const std::uint32_t* words = nullptr;
+};
+
+int32_t region_image(bfn_workspace ws, std::uint32_t query, bool predecessors, RegionImage& image) {
   const std::uint32_t p0 = ws->h_tile_off[query], slots = ws->h_tile_off[query + 1] - p0;
   const auto& toff = ws->graph->h_tile_off;
+  auto& offsets = image.offsets;
   offsets.resize(slots + 1ull);
   offsets[0] = 0;
   for (std::uint32_t i = 0; i < slots; ++i) {
@@ -1296,42 +1303,55 @@ int32_t region_image(bfn_workspace ws, std::uint32_t query, bool predecessors,
   const std::uint64_t n = offsets[slots];
   const std::size_t head = align_up(8ull * slots, 256);
   BFN_HIP(ws->region.reserve(head + 4ull * std::max<std::uint64_t>(n, 1)));
-  BFN_HIP(ws->h_region.reserve(head + 4ull * std::max<std::uint64_t>(n, 1)));
+  const void* upload = offsets.data();
+  std::uint32_t* words = nullptr;
+  if (ws->h_region.reserve(head + 4ull * std::max<std::uint64_t>(n, 1)) == hipSuccess) {
+    std::memcpy(ws->h_region.ptr, offsets.data(), 8ull * slots);
+    upload = ws->h_region.ptr;
+    words = reinterpret_cast<std::uint32_t*>(ws->h_region.as<char>() + head);
+  } else {
+    (void)hipGetLastError();
+    image.plain.resize(n);
+    words = image.plain.data();
+  }
   hipStream_t s = ws->stream;
-  std::memcpy(ws->h_region.ptr, offsets.data(), 8ull * slots);
-  BFN_HIP(hipMemcpyAsync(ws->region.ptr, ws->h_region.ptr, 8ull * slots, hipMemcpyHostToDevice, s));
+  const unsigned long long* at = nullptr;  // one run of tiles needs no offsets on the device
+  if (ws->h_tiles[p0 + slots - 1] - ws->h_tiles[p0] != slots - 1) {
+    BFN_HIP(hipMemcpyAsync(ws->region.ptr, upload, 8ull * slots, hipMemcpyHostToDevice, s));
+    at = ws->region.as<unsigned long long>();
+  }
   const DevControl* c = ws->h_control.as<DevControl>();
   const std::uint32_t copy = c->rounds_executed & 1u;
-  const unsigned long long* at = ws->region.as<unsigned long long>();
   std::uint32_t* out = reinterpret_cast<std::uint32_t*>(ws->region.as<char>() + head);
   BFN_HIP(predecessors
               ? predecessors_launch(ws->graph->view, ws->view, query, slots, copy, at, out, s)
               : gather_region_launch(ws->graph->view, ws->view, query, slots, copy, at, out, s));
-  if (n)
-    BFN_HIP(hipMemcpyAsync(ws->h_region.as<char>() + head, out, 4ull * n, hipMemcpyDeviceToHost, s));
+  if (n) BFN_HIP(hipMemcpyAsync(words, out, 4ull * n, hipMemcpyDeviceToHost, s));
   BFN_HIP(hipStreamSynchronize(s));
-  *image = reinterpret_cast<const std::uint32_t*>(ws->h_region.as<char>() + head);
+  image.words = words;
   return BFN_OK;
 }
 
 // The image over the whole graph, `none` outside the query's tiles.  Only
 // the region crosses from the device; the caller's array is written once, in
-// vertex order, on the host.  1M vertices, against one pageable copy of an
-// image scattered on the device: 576 of 4096 tiles selected 265 -> 90 us,
-// all of them 260 us both ways.
+// vertex order, on the host, a copy per run of consecutive tiles.  Against
+// one pageable copy of an image scattered on the device: 64 of 4096 tiles of
+// 256 vertices 263 -> 57 us, all of them 260 -> 234; 4096 of 16384 tiles of
+// 512 1928 -> 802, all of them 1926 -> 1750 (a copy per tile took 2237).
 int32_t graph_image(bfn_workspace ws, std::uint32_t query, bool predecessors, std::uint32_t none,
                     std::uint32_t* out) {
-  std::vector<unsigned long long> offsets;
-  const std::uint32_t* image = nullptr;
-  if (int32_t rc = region_image(ws, query, predecessors, offsets, &image)) return rc;
+  RegionImage image;
+  if (int32_t rc = region_image(ws, query, predecessors, image)) return rc;
   const auto& toff = ws->graph->h_tile_off;
   const std::uint32_t p0 = ws->h_tile_off[query], p1 = ws->h_tile_off[query + 1];
   std::uint32_t v = 0;
-  for (std::uint32_t p = p0; p < p1; ++p) {
-    const std::uint32_t T = ws->h_tiles[p];
-    std::fill(out + v, out + toff[T], none);
-    std::memcpy(out + toff[T], image + offsets[p - p0], 4ull * (toff[T + 1] - toff[T]));
-    v = toff[T + 1];
+  for (std::uint32_t p = p0, run = p; p < p1; p = run) {
+    do ++run;
+    while (run < p1 && ws->h_tiles[run] == ws->h_tiles[run - 1] + 1);
+    const std::uint32_t begin = toff[ws->h_tiles[p]], end = toff[ws->h_tiles[run - 1] + 1];
+    std::fill(out + v, out + begin, none);
+    std::memcpy(out + begin, image.words + image.offsets[p - p0], 4ull * (end - begin));
+    v = end;
   }
   std::fill(out + v, out + ws->graph->V, none);
   return BFN_OK;
@@ -1357,10 +1377,9 @@ int32_t bfn_batch_region_distances(bfn_workspace ws, uint32_t query, float* out,
   *count = n;
   if (!out) return BFN_OK;
   if (capacity < n) return fail(BFN_E_INVALID_ARGUMENT, "output capacity too small");
-  std::vector<unsigned long long> offsets;
-  const std::uint32_t* image = nullptr;
-  if (int32_t rc = region_image(ws, query, false, offsets, &image)) return rc;
-  std::memcpy(out, image, 4ull * n);
+  RegionImage image;
+  if (int32_t rc = region_image(ws, query, false, image)) return rc;
+  std::memcpy(out, image.words, 4ull * n);
   return BFN_OK;
 }
 

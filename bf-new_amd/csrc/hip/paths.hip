@@ -334,8 +334,18 @@ __global__ __launch_bounds__(512) void compact_paths_kernel(PathArgs a) {
   }
 }
 
+// Where the image of a query's region holds its position i, tile T: at
+// offsets[i], or, where the tiles are one run (no offsets), as far from the
+// first tile as in the graph.
+__device__ __forceinline__ unsigned long long region_at(const DevGraph& g, const DevBatch& b, std::uint32_t q,
+                                                        const unsigned long long* offsets, std::uint32_t i,
+                                                        std::uint32_t T) {
+  if (offsets) return offsets[i];
+  return g.tile_vertex_offsets[T] - g.tile_vertex_offsets[b.tiles[slot_at(b, b.tile_begin[q])]];
+}
+
 // Smallest-EdgeId tight admitted predecessor of each vertex of query q, tile
-// by tile in the order of its sorted selected tiles (tile i at offsets[i]).
+// by tile in the order of its sorted selected tiles.
 __global__ void predecessors_kernel(DevGraph g, DevBatch b, std::uint32_t q,
                                     std::uint32_t jacobi_copy, const unsigned long long* offsets,
                                     std::uint32_t* out) {
@@ -345,6 +355,7 @@ __global__ void predecessors_kernel(DevGraph g, DevBatch b, std::uint32_t q,
   const std::uint32_t T = b.tiles[s];
   const std::uint32_t v0 = g.tile_vertex_offsets[T];
   const std::uint32_t npt = g.tile_vertex_offsets[T + 1] - v0;
+  const unsigned long long at = region_at(g, b, q, offsets, blockIdx.x, T);
   const std::uint32_t in0 = g.in_nbr_offsets[T];
   const std::uint32_t col = column_of(b, q, jacobi_copy);
   for (std::uint32_t i = threadIdx.x; i < npt; i += blockDim.x) {
@@ -369,7 +380,7 @@ __global__ void predecessors_kernel(DevGraph g, DevBatch b, std::uint32_t q,
         }
       }
     }
-    out[offsets[blockIdx.x] + i] = best_u;
+    out[at + i] = best_u;
   }
 }
 
@@ -533,7 +544,7 @@ hipError_t predecessors_launch(const DevGraph& g, const DevBatch& b, std::uint32
 }
 
 // Copies query q's final labels tile by tile, in the order of its sorted
-// selected tiles, to out[offsets[i] ...] (i = position within the query).
+// selected tiles, tile by tile.
 __global__ void gather_region_kernel(DevGraph g, DevBatch b, std::uint32_t q,
                                      std::uint32_t jacobi_copy, const unsigned long long* offsets,
                                      std::uint32_t* out) {
@@ -545,7 +556,7 @@ __global__ void gather_region_kernel(DevGraph g, DevBatch b, std::uint32_t q,
   const std::uint32_t npt = g.tile_vertex_offsets[T + 1] - g.tile_vertex_offsets[T];
   const std::uint32_t* src =
       b.dist + b.slot_dist[s] + static_cast<unsigned long long>(column_of(b, q, jacobi_copy)) * npt;
-  std::uint32_t* dst = out + offsets[i];
+  std::uint32_t* dst = out + region_at(g, b, q, offsets, i, T);
   for (std::uint32_t k = threadIdx.x; k < npt; k += blockDim.x) dst[k] = src[k];
 }
 

@@ -16,6 +16,7 @@ sys.path.insert(0, TESTS)
 import numpy as np  # noqa: E402
 
 import bfnew_amd as bfn  # noqa: E402
+import oracle  # noqa: E402
 
 bfn.HIP_LIB_PATH = sys.argv[1]
 
@@ -141,6 +142,38 @@ def costs(dev):
     check(refused(lambda: dg.update_node_costs(bad)) == 1, "NaN costs accepted")
     largest(DEVICE, 1 << 40)
     expect_weights(dev, dg, view, base + half)
+    dg.close()
+
+
+def images(dev):
+    """Label and predecessor images of a run of tiles, of tiles apart and of
+    the whole graph, with pinned memory for them and without."""
+    hg, dg = graph(dev, 9, 8, 33)
+    view = hg.view()
+    T = 72
+    regions = [np.arange(T, dtype=np.uint32), np.arange(20, 31, dtype=np.uint32),
+               np.array([0, 1, 2, 9, 10, 18, 70, 71], np.uint32), np.array([33], np.uint32)]
+    sources = [[int(r[len(r) // 2]) * 33 + 4] for r in regions]
+    ws = bfn.Workspace(dev)
+    ws.submit(dg, bfn.Batch(sources, [[s[0] + 1] for s in sources], regions),
+              bfn.run_options(engine=bfn.FRONTIER_PUSH, control_mode=bfn.CHUNKED), bfn.tuning(tile_sweeps=0))
+    first = []
+    for pinned in (1 << 40, 0):
+        for q in (3, 2, 1, 0):  # growing, so that none fits what an earlier one took
+            largest(PINNED, pinned)
+            want, _ = oracle_query(view, sources[q], regions[q])
+            where = oracle.region_vertices(view["tile_vertex_offsets"], regions[q])
+            check(np.array_equal(bits(ws.distances(q)), bits(want)), f"labels of {q}, pinned {pinned}")
+            check(np.array_equal(bits(ws.region_distances(q)), bits(want[where])), f"region of {q}")
+            first.append(ws.predecessors(q))
+        ws.close()
+        largest(PINNED, 1 << 40)
+        ws = bfn.Workspace(dev)
+        ws.submit(dg, bfn.Batch(sources, [[s[0] + 1] for s in sources], regions),
+                  bfn.run_options(engine=bfn.FRONTIER_PUSH, control_mode=bfn.CHUNKED), bfn.tuning(tile_sweeps=0))
+    for a, b in zip(first[:4], first[4:]):
+        check(np.array_equal(a, b), "predecessors with and without pinned memory")
+    ws.close()
     dg.close()
 
 
