@@ -270,10 +270,12 @@ struct QueryStatusDev {
 };
 
 // Bits of PathArgs::query_clean: the query converged without error; pass 1
-// walked one of its targets with backtracking (its frames hold only the last
-// walk, so pass 2 walks again).
+// walked one of its several targets with backtracking (the frames hold only
+// the last walk, so pass 2 walks again); or its one target (the frames hold
+// that walk, without labels).
 constexpr std::uint32_t kPathClean = 1u;
 constexpr std::uint32_t kPathGeneral = 2u;
+constexpr std::uint32_t kPathKept = 4u;
 
 // Arguments of the compact-path passes.
 struct PathArgs {
@@ -302,6 +304,7 @@ struct PathArgs {
   std::uint32_t* host_vertices;         // pinned copies of the arenas, or null
   std::uint32_t* host_labels;
   std::uint32_t* host_edges;
+  std::uint32_t* host_left;             // pass 2: set instead of walking kPathGeneral queries again, or null
   const std::uint32_t* query_list;      // queries to reconstruct (null: all)
   std::uint32_t jacobi_copy_from_control;  // take the column from round parity
   std::uint32_t pad2;

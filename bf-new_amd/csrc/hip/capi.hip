@@ -179,7 +179,8 @@ struct bfn_workspace_s {
   const unsigned long long* frame_base_ptr = nullptr;  // in `meta`
   bool submitted = false, completed = false, have_paths = false;
   bool paths_counted = false;  // summaries and offsets of this completion's paths are on the host
-  bool paths_emitted = false;  // and the paths themselves in h_arena
+  bool paths_emitted = false;  // and the paths themselves in the arenas
+  bool arena_pinned = false;   // h_arena has room for the arenas' copies
   bool slots_resolved = false; // the batch's neighbour slots and descriptors are on the device
   std::uint64_t arena_vertices = 0, arena_room = 0;
   std::uint32_t most_targets = 0;
@@ -1404,7 +1405,7 @@ int32_t bfn_batch_paths(bfn_workspace ws, bfn_target_summary* summaries, uint64_
   BFN_HIP(ws->paths_len.reserve(8ull * NT));
   BFN_HIP(ws->frames.reserve(12ull * std::max<std::uint64_t>(ws->frame_words, 1)));
   BFN_HIP(ws->onpath.reserve(4ull * std::max<std::uint64_t>(ws->pool_words, 1)));
-  BFN_HIP(ws->h_paths.reserve(out_bytes));
+  BFN_HIP(ws->h_paths.reserve(out_bytes + sizeof(std::uint32_t)));
   char* hp = ws->h_paths.as<char>();
   PathArgs a{};
   a.g = ws->graph->view;
@@ -1442,46 +1443,66 @@ int32_t bfn_batch_paths(bfn_workspace ws, bfn_target_summary* summaries, uint64_
     ws->path_stamp += NT;
     return hipSuccess;
   };
-  // Room for `vertices` path vertices on the device and in pinned memory.
+  // Room for `vertices` path vertices on the device, and for copies of them in
+  // pinned memory where that can be had.
   auto make_room = [&](std::uint64_t vertices) -> hipError_t {
     if (vertices <= ws->arena_room) return hipSuccess;
     ws->arena_room = 0;
-    hipError_t e = ws->arena_v.reserve(4ull * vertices);
-    if (e == hipSuccess) e = ws->arena_l.reserve(4ull * vertices);
-    if (e == hipSuccess) e = ws->arena_e.reserve(4ull * vertices);
-    if (e == hipSuccess) e = ws->h_arena.reserve(12ull * vertices);
-    if (e == hipSuccess) ws->arena_room = vertices;
-    return e;
+    ws->arena_pinned = false;
+    hipError_t e = hipSuccess;
+    for (DeviceBuffer* d : {&ws->arena_v, &ws->arena_l, &ws->arena_e})
+      if (e == hipSuccess) e = d->reserve(4ull * vertices);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      return e;
+    }
+    ws->arena_room = vertices;
+    ws->arena_pinned = ws->h_arena.reserve(12ull * vertices) == hipSuccess;
+    if (!ws->arena_pinned) (void)hipGetLastError();
+    return hipSuccess;
   };
   // Pass 2 writes the paths to the device arenas (what occupancy counts) and
   // to pinned host memory, where a path's few hundred bytes cost less than
-  // three copies.
-  auto emit = [&]() -> hipError_t {
+  // three copies.  With `early` it leaves queries that have to be walked again
+  // and says so in h_paths.
+  std::uint32_t* left = reinterpret_cast<std::uint32_t*>(hp + out_bytes);
+  auto emit = [&](bool early) -> hipError_t {
     hipError_t e = take_stamps();
     if (e != hipSuccess) return e;
+    *left = 0;
     a.pass = 2;
+    a.host_left = early ? left : nullptr;
     a.arena_capacity = ws->arena_room;
     a.arena_vertices = ws->arena_v.as<std::uint32_t>();
     a.arena_labels = ws->arena_l.as<std::uint32_t>();
     a.arena_edges = ws->arena_e.as<std::uint32_t>();
-    a.host_vertices = ws->h_arena.as<std::uint32_t>();
-    a.host_labels = a.host_vertices + ws->arena_room;
-    a.host_edges = a.host_labels + ws->arena_room;
+    if (ws->arena_pinned) {
+      a.host_vertices = ws->h_arena.as<std::uint32_t>();
+      a.host_labels = a.host_vertices + ws->arena_room;
+      a.host_edges = a.host_labels + ws->arena_room;
+    }
     return paths_launch(a, ws->Q, s);
   };
-  // Both passes run once per completed batch, pass 2 in the room that earlier
-  // paths had (or 64 vertices per target): the second call, the one that
-  // brings the arenas, finds the paths on the host unless they needed more.
+  // Pass 1 runs once per completed batch, and pass 2 behind the same wait, in
+  // the room that earlier paths had (or 64 vertices per target): the call that
+  // brings the arenas then finds the paths on the host.  A call without arenas
+  // does not wait for walks that pass 2 would have to repeat (64 queries with
+  // four targets each on 32x32x64 tiles, 6 % of the nodes without cost:
+  // summaries 316 -> 183 us), and does without pass 2 where there is no memory
+  // for it.
   if (!ws->paths_counted) {
-    BFN_HIP(make_room(std::min<std::uint64_t>(64ull * NT, 1ull << 20)));
+    const bool wanted = vertices && labels && edge_ids;
+    const bool emitting =
+        make_room(std::min<std::uint64_t>(64ull * NT, 1ull << 20)) == hipSuccess && ws->arena_pinned;
     BFN_HIP(take_stamps());
     BFN_HIP(paths_launch(a, ws->Q, s));
     BFN_HIP(scan_u64_launch(a.lengths, offsets, NT, s));
-    BFN_HIP(emit());
+    if (emitting) BFN_HIP(emit(!wanted));
     BFN_HIP(hipMemcpyAsync(hp, ws->paths_out.ptr, out_bytes, hipMemcpyDeviceToHost, s));
     BFN_HIP(hipStreamSynchronize(s));
     ws->paths_counted = true;
-    ws->paths_emitted = reinterpret_cast<const std::uint64_t*>(hp + off_at)[NT] <= ws->arena_room;
+    ws->paths_emitted = emitting && *left == 0 &&
+                        reinterpret_cast<const std::uint64_t*>(hp + off_at)[NT] <= ws->arena_room;
   }
   std::memcpy(summaries, hp, 28ull * NT);
   std::memcpy(path_offsets, hp + off_at, 8ull * (NT + 1));
@@ -1491,15 +1512,22 @@ int32_t bfn_batch_paths(bfn_workspace ws, bfn_target_summary* summaries, uint64_
   if (!vertices || !labels || !edge_ids) return fail(BFN_E_INVALID_ARGUMENT, "arenas must all be given");
   if (arena_capacity < total) return fail(BFN_E_INVALID_ARGUMENT, "arena capacity too small");
   if (!ws->paths_emitted) {
-    BFN_HIP(make_room(total + total / 4));
-    BFN_HIP(emit());
+    if (make_room(total + total / 4) != hipSuccess) BFN_HIP(make_room(std::max<std::uint64_t>(total, 1)));
+    BFN_HIP(emit(false));
     BFN_HIP(hipStreamSynchronize(s));
     ws->paths_emitted = true;
   }
-  const std::uint32_t* ha = ws->h_arena.as<std::uint32_t>();
-  std::memcpy(vertices, ha, 4ull * total);
-  std::memcpy(labels, ha + ws->arena_room, 4ull * total);
-  std::memcpy(edge_ids, ha + 2 * ws->arena_room, 4ull * total);
+  if (ws->arena_pinned) {
+    const std::uint32_t* ha = ws->h_arena.as<std::uint32_t>();
+    std::memcpy(vertices, ha, 4ull * total);
+    std::memcpy(labels, ha + ws->arena_room, 4ull * total);
+    std::memcpy(edge_ids, ha + 2 * ws->arena_room, 4ull * total);
+  } else if (total) {
+    BFN_HIP(hipMemcpyAsync(vertices, ws->arena_v.ptr, 4ull * total, hipMemcpyDeviceToHost, s));
+    BFN_HIP(hipMemcpyAsync(labels, ws->arena_l.ptr, 4ull * total, hipMemcpyDeviceToHost, s));
+    BFN_HIP(hipMemcpyAsync(edge_ids, ws->arena_e.ptr, 4ull * total, hipMemcpyDeviceToHost, s));
+    BFN_HIP(hipStreamSynchronize(s));
+  }
   ws->have_paths = true;
   ws->arena_vertices = total;
   return BFN_OK;

@@ -285,6 +285,10 @@ __global__ __launch_bounds__(512) void compact_paths_kernel(PathArgs a) {
   const bool emit = a.pass == 2;
   if (emit && a.arena_capacity != ~0ull && a.offsets[a.target_total] > a.arena_capacity)
     return;  // the host retries with room for them
+  if (emit && a.host_left && (state & kPathGeneral)) {
+    if (threadIdx.x == 0) *a.host_left = 1u;
+    return;
+  }
   __shared__ std::uint32_t general;  // targets for walk_backtracking
   if (threadIdx.x == 0) general = 0;
   __syncthreads();
@@ -294,7 +298,7 @@ __global__ __launch_bounds__(512) void compact_paths_kernel(PathArgs a) {
       const unsigned long long frames = fb + room * (t - t0);
       if (emit) {
         const std::int32_t n = static_cast<std::int32_t>(a.lengths[t]);
-        if (n) copy_out(t, n - 1, frames, true);
+        if (n) copy_out(t, n - 1, frames, !(state & kPathKept));
         continue;
       }
       const std::uint32_t dt = label_of(g, b, q, target, copy, nullptr);
@@ -315,7 +319,8 @@ __global__ __launch_bounds__(512) void compact_paths_kernel(PathArgs a) {
     wave_fence();
     __syncthreads();
     if (emit) return;
-    const std::uint32_t marked = general ? state | kPathGeneral : state & ~kPathGeneral;
+    const std::uint32_t again = general == 0 ? 0u : t1 - t0 == 1 ? kPathKept : kPathGeneral;
+    const std::uint32_t marked = (state & kPathClean) | again;
     if (threadIdx.x == 0 && marked != state) a.query_clean[q] = marked;
     if (general == 0) return;
   }

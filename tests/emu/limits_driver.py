@@ -20,7 +20,7 @@ import oracle  # noqa: E402
 
 bfn.HIP_LIB_PATH = sys.argv[1]
 
-from helpers import bits, oracle_query  # noqa: E402
+from helpers import bits, expected_paths, oracle_query, path_failures, with_node_costs  # noqa: E402
 
 DEVICE, PINNED = 0, 1
 FAILURES = []
@@ -173,6 +173,73 @@ def images(dev):
                   bfn.run_options(engine=bfn.FRONTIER_PUSH, control_mode=bfn.CHUNKED), bfn.tuning(tile_sweeps=0))
     for a, b in zip(first[:4], first[4:]):
         check(np.array_equal(a, b), "predecessors with and without pinned memory")
+    ws.close()
+    dg.close()
+
+
+def paths(dev):
+    """Compact paths, some of them over zero-cost plateaus, as two calls (the
+    first without arenas) and as one, with memory to write the paths early and
+    without."""
+    hg, dg = graph(dev, 9, 8, 32)
+    rng = np.random.default_rng(2)
+    costs = hg.view()["node_costs"].copy()
+    costs[rng.random(len(costs)) < 0.05] = 0.0
+    dg.update_node_costs(costs)
+    view = with_node_costs(hg.view(), costs)
+    tiles = np.arange(18, dtype=np.uint32)
+    targets = sorted(int(v) for v in rng.choice(18 * 32, 60, False))
+    want = expected_paths(view, [5], targets, tiles)
+    walks = [w[1:] for w in want[1]]
+    batch = bfn.Batch([[5]], [targets], [tiles])
+    total = sum(len(v) for v, _ in walks)
+    for device, pinned in ((1 << 40, 1 << 40), (12000, 1 << 40), (1 << 40, 4000)):
+        for arenas_at_once in (False, True):
+            what = (device, pinned, arenas_at_once)
+            ws = bfn.Workspace(dev)
+            ws.submit(dg, batch, bfn.run_options(engine=bfn.FRONTIER_PUSH, control_mode=bfn.CHUNKED),
+                      bfn.tuning(tile_sweeps=0))
+            largest(DEVICE, device)
+            largest(PINNED, pinned)
+            summaries = (bfn.TargetSummary * 60)()
+            offsets, n = np.zeros(61, np.uint64), ctypes.c_uint64()
+            out = [np.zeros(total, t) for t in (np.uint32, np.float32, np.uint32)]
+            f, p = bfn.hip_lib().bfn_batch_paths, lambda a: a.ctypes.data_as(ctypes.c_void_p)
+            if not arenas_at_once:
+                rc = f(ws.h, summaries, p(offsets), None, None, None, 0, ctypes.byref(n))
+                check(rc == 0 and n.value == total, f"summaries {what}: {rc}, {n.value} of {total} vertices")
+            rc = f(ws.h, summaries, p(offsets), *(p(a) for a in out), total, ctypes.byref(n))
+            check(rc == 0 and n.value == total, f"arenas {what}: {rc}")
+            arrays = dict(summaries=np.ctypeslib.as_array(summaries), offsets=offsets, vertices=out[0],
+                          labels=out[1], edge_ids=out[2])
+            check(rc or path_failures(arrays, [want]) == [], f"paths {what}")
+            largest(DEVICE, 1 << 40)
+            largest(PINNED, 1 << 40)
+            occupancy = np.zeros(view["vertex_count"], np.int32)
+            for verts, _ in walks:
+                occupancy[verts] += 1
+            if rc == 0:
+                check(np.array_equal(ws.occupancy(), occupancy), f"occupancy {what}")
+            ws.close()
+    dg.close()
+
+
+def long_paths(dev):
+    """Paths of more vertices than the room first made for them, on positive
+    costs (tests/test_gpu_path_walks.py on a shorter strip)."""
+    hg, dg = graph(dev, 300, 1, 4)
+    view = with_node_costs(hg.view(), hg.view()["node_costs"])
+    tiles = np.arange(300, dtype=np.uint32)
+    targets = [1150, 1171, 1199]
+    want = [expected_paths(view, [1], targets, tiles)]
+    ws = bfn.Workspace(dev)
+    ws.submit(dg, bfn.Batch([[1]], [targets], [tiles]),
+              bfn.run_options(engine=bfn.FRONTIER_PUSH, control_mode=bfn.CHUNKED), bfn.tuning(tile_sweeps=0))
+    for _ in range(2):
+        arrays = ws.path_arrays()
+        check(arrays["offsets"][-1] > 64 * 3, f"{arrays['offsets'][-1]} vertices")
+        check(path_failures(arrays, want) == [], "paths")
+        ws.rerun()
     ws.close()
     dg.close()
 

@@ -106,3 +106,36 @@ def oracle_region(view, layout, source, tiles):
     """Oracle Dijkstra labels of one query, in the region (tile by tile) order."""
     d, _ = oracle_query(view, [source], tiles)
     return d[oracle.region_vertices(layout["tile_vertex_offsets"], tiles)]
+
+
+def with_node_costs(view, costs):
+    """The view under other node costs: an edge weighs its head's cost."""
+    heads = np.repeat(np.arange(len(costs)), np.diff(view["column_offsets"].astype(np.int64)))
+    return dict(view, node_costs=costs, weights=costs[view["destinations"]], in_weights=costs[heads])
+
+
+def expected_paths(view, sources, targets, tiles):
+    """The oracle's labels of one query and, per target, its reconstruction
+    (outcome, vertices, edge ids)."""
+    labels, _ = oracle_query(view, sources, tiles)
+    sel = tile_mask(view["tile_count"], tiles)
+    return labels, [oracle.reconstruct(view["vertex_count"], view["column_offsets"], view["sources"],
+                                       view["in_weights"], view["in_edge_ids"], view["owner_tiles"],
+                                       sel, labels, sources, t) for t in targets]
+
+
+def path_failures(arrays, queries):
+    """Compares Workspace.path_arrays() of a batch with its queries'
+    expected_paths(); the targets that differ."""
+    failures, at = [], 0
+    for q, (labels, walks) in enumerate(queries):
+        for what, verts, edges in walks:
+            lo, hi = int(arrays["offsets"][at]), int(arrays["offsets"][at + 1])
+            s = arrays["summaries"][at]
+            at += 1
+            if (int(s["reconstruction"]) != {"complete": 0, "unreachable": 1, "no_tight_path": 3}[what] or
+                    list(arrays["vertices"][lo:hi]) != list(verts) or
+                    list(arrays["edge_ids"][lo:max(lo, hi - 1)]) != list(edges) or
+                    not np.array_equal(bits(arrays["labels"][lo:hi]), bits(labels[verts]))):
+                failures.append((q, int(s["target"])))
+    return failures

@@ -16,7 +16,7 @@ sys.path.insert(0, os.path.join(HERE, "emu"))
 import build_emu  # noqa: E402
 
 
-@pytest.mark.parametrize("check", ["estimate", "server", "costs", "images"])
+@pytest.mark.parametrize("check", ["estimate", "server", "costs", "images", "paths", "long_paths"])
 def test_emulated_limits(check):
     lib = build_emu.build()
     env = dict(os.environ)

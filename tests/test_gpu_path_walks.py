@@ -8,7 +8,7 @@ import pytest
 
 import bfnew_amd as bfn
 import oracle
-from helpers import bits, oracle_query, tile_mask
+from helpers import bits, expected_paths, oracle_query, path_failures, tile_mask, with_node_costs
 
 pytestmark = pytest.mark.gpu
 
@@ -61,4 +61,56 @@ def test_path_walks(device, zero_share, nodes, targets):
                     assert np.array_equal(bits(p["labels"]), bits(labels[verts])), label
             ws.rerun()
         ws.close()
+    dg.close()
+
+
+def test_paths_longer_than_the_first_room(device):
+    """Paths of more than 64 vertices per target on positive costs: pass 2 has
+    no room at first, and the paths are copied out of the frames that pass 1
+    left; then room that an earlier batch grew."""
+    hg = bfn.HostGraph.synthetic(400, 1, 4, 5, host_graph=True)
+    dg = bfn.DeviceGraph(device, hg.layout())
+    view = with_node_costs(hg.view(), hg.view()["node_costs"])
+    assert view["node_costs"].min() > 0.0
+    tiles = np.arange(400, dtype=np.uint32)
+    sources, targets = [[1], [0, 6]], [[1502, 1540, 1571, 1599], [1450, 1588]]
+    want = [expected_paths(view, s, t, tiles) for s, t in zip(sources, targets)]
+    for engine in (bfn.JACOBI_PULL, bfn.FRONTIER_PUSH):
+        ws = bfn.Workspace(device)
+        ws.submit(dg, bfn.Batch(sources, targets, [tiles] * 2),
+                  bfn.run_options(engine=engine, control_mode=bfn.CHUNKED),
+                  bfn.tuning(tile_sweeps=0, boundary_mode=1))
+        for _ in range(2):
+            arrays = ws.path_arrays()
+            assert arrays["offsets"][-1] > 64 * 6
+            assert path_failures(arrays, want) == [], engine
+            ws.rerun()
+        ws.close()
+    dg.close()
+
+
+@pytest.mark.parametrize("zero_share", [0.03, 0.08])
+def test_plateaus_of_many_queries(device, zero_share):
+    """Batches where some queries have to be walked again by pass 2 and others
+    do not: the first call leaves the former to the second."""
+    hg = bfn.HostGraph.synthetic(24, 24, 32, 5, host_graph=True)
+    dg = bfn.DeviceGraph(device, hg.layout())
+    costs = hg.view()["node_costs"].copy()
+    costs[np.random.default_rng(3).random(len(costs)) < zero_share] = 0.0
+    dg.update_node_costs(costs)
+    view = with_node_costs(hg.view(), costs)
+    qs = hg.synthetic_queries(20, seed=4, side_min=2, side_max=6)
+    tiles = [hg.query_tiles(q) for q in qs]
+    want = [expected_paths(view, [q.source], [q.target], t) for q, t in zip(qs, tiles)]
+    plateau = [any(labels[v] == labels[u] for v, u in zip(verts, verts[1:]))
+               for labels, ((_, verts, _),) in want]
+    assert any(plateau) and not all(plateau)
+    ws = bfn.Workspace(device)
+    ws.submit(dg, bfn.Batch([[q.source] for q in qs], [[q.target] for q in qs], tiles),
+              bfn.run_options(engine=bfn.FRONTIER_PUSH, control_mode=bfn.CHUNKED),
+              bfn.tuning(tile_sweeps=0, boundary_mode=1))
+    for _ in range(2):
+        assert path_failures(ws.path_arrays(), want) == []
+        ws.rerun()
+    ws.close()
     dg.close()
