@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 
 import bfnew_amd as bfn
-from helpers import oracle_query
+from helpers import expected_paths, oracle_query, with_node_costs
 
 pytestmark = pytest.mark.gpu
 
@@ -84,6 +84,37 @@ def test_server_results_equal_alone_and_oracle(device, engine):
     assert len(got) == len(qs), f"{len(got)} of {len(qs)} responses"
     assert stats["completed"] == len(qs)
     _check_against_alone_and_oracle(device, dg, view, engine, qs, tiles, got)
+
+
+@pytest.mark.parametrize("engine", [bfn.FRONTIER_PUSH, bfn.JACOBI_PULL])
+def test_server_plateaus(device, engine):
+    """Paths over zero-cost plateaus need backtracking: more requests than
+    places, so that a place serves such a request before and after others."""
+    hg, dg = _graph(device)
+    costs = hg.view()["node_costs"].copy()
+    costs[np.random.default_rng(3).random(len(costs)) < 0.03] = 0.0
+    dg.update_node_costs(costs)
+    view = with_node_costs(hg.view(), costs)
+    qs = hg.synthetic_queries(48, seed=8, side_min=2, side_max=8)
+    tiles = [hg.query_tiles(q) for q in qs]
+    want = [expected_paths(view, [q.source], [q.target], t) for q, t in zip(qs, tiles)]
+    over = [any(ref[u] == ref[v] for u, v in zip(verts, verts[1:])) for ref, ((_, verts, _),) in want]
+    assert any(over[:24]) and any(over[24:]) and not all(over[:24]) and not all(over[24:])
+    print(f"server plateaus engine={engine}", flush=True)
+    server = bfn.Server(device, dg, budget_bytes=64 << 20, max_active_queries=4,
+                        rounds_per_chunk=2, engine=engine, tile_sweeps=0)
+    try:
+        for i, q in enumerate(qs):
+            server.submit(i, q.source, q.target, tiles[i])
+        got = _drain(server, len(qs))
+    finally:
+        server.close()
+    assert len(got) == len(qs), f"{len(got)} of {len(qs)} responses"
+    for i, (q, (ref, ((_, verts, edges),))) in enumerate(zip(qs, want)):
+        assert np.float32(got[i]["distance"]) == np.float32(ref[q.target]), i
+        assert list(got[i]["vertices"]) == list(verts), i
+        assert list(got[i]["edge_ids"]) == list(edges), i
+    dg.close()
 
 
 @pytest.mark.timeout(600)
