@@ -217,7 +217,8 @@ __device__ __forceinline__ void visit_pull(const DevGraph& g, const DevBatch& b,
   __syncthreads();
   // Stage the read column of every in-neighbour slab (k = 0 is T itself).  A
   // wave takes four slabs at a time and keeps two 64-word rows of each in
-  // flight, so a list of up to 16 small slabs costs one round trip.
+  // flight, so 4 * B / 64 slabs of up to 128 words (16 at 256 threads) cost
+  // one round trip.
   constexpr std::uint32_t kSlabs = 4, kRows = 2, kWaves = B / 64;
   const std::uint32_t lane = tid & 63u, wave = tid >> 6;
   const bool one_by_one = slab_by_slab<B, kSlabs, kRows>(K, npt);
@@ -739,8 +740,8 @@ __device__ __forceinline__ void process_round(const DevGraph& g, const DevBatch&
   auto visit = [&](std::uint32_t s) {
     const SlotDesc d = load_slot_desc(g, b, s);
     bool run = true;
-    // A variant without the slot's engine cannot visit it; prep_slots_kernel
-    // flags such a batch (the host picks the variant from the batch's
+    // A variant without the slot's engine cannot visit it; seed_kernel flags
+    // such a batch (the host picks the variant from the batch's
     // engines, so it does not happen).  Nothing is done here: any extra
     // global operation on this path costs the variant 18 VGPRs.
     if (d.engine == kJacobiPull) {
