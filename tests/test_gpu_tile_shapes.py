@@ -79,3 +79,27 @@ def test_tile_shapes_bit_exact(device, nodes, block):
             assert np.array_equal(bits(ws.distances(i)), bits(want[i])), (c, i)
         ws.close()
     dg.close()
+
+
+@pytest.mark.parametrize("sources", [1, 63, 64, 65, 300])
+def test_many_sources_bit_exact(device, sources):
+    """Sources of one query are taken by the lanes of a wave, several of them in
+    one tile."""
+    hg = bfn.HostGraph.synthetic(9, 8, 33, 7, host_graph=True)
+    view = hg.view()
+    dg = bfn.DeviceGraph(device, hg.layout())
+    rng = np.random.default_rng(sources)
+    tiles = np.arange(72, dtype=np.uint32)
+    batch = bfn.Batch([sorted(int(v) for v in rng.choice(72 * 33, n, False)) for n in (sources, 2)],
+                      [[7], [11]], [tiles] * 2)
+    want = [oracle_query(view, s, tiles)[0] for s in batch.sources]
+    for c in CONFIGS:
+        ws = bfn.Workspace(device)
+        ws.submit(dg, batch, bfn.run_options(engine=c["engine"], control_mode=c["control"]),
+                  bfn.tuning(tile_sweeps=c["sweeps"], boundary_mode=c["boundary"],
+                             push_window=c.get("window", 0.0)))
+        assert ws.status()[0].converged == 1, c
+        for i in range(2):
+            assert np.array_equal(bits(ws.distances(i)), bits(want[i])), (c, i)
+        ws.close()
+    dg.close()
